@@ -182,6 +182,12 @@ struct Space {
     DBuf<int32_t> elems;
   };
   std::map<uint64_t, std::unique_ptr<BndSet>> bnd_sets;
+  // load vectors (H1): per dof its entries among the element values (local dof * nel + element,
+  // increasing) and the values (nloc x nel) they are summed from, built on first use; the kernels
+  // of one space all run on its context's stream
+  DBuf<uint32_t> d_lptr;  // ndof+1
+  DBuf<uint32_t> d_lent;  // nel*nloc
+  DBuf<double> d_lin;     // nloc*nel
   // cached kernel tables keyed by a signature
   std::map<std::string, DBuf<double> *> tables;
   ~Space() {

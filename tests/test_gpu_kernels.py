@@ -1,0 +1,80 @@
+"""Kernels at the sizes where they can go wrong: tile edges, remainders, the smallest problems.
+
+Each is compared with the CPU oracle (or numpy) in FP64.
+"""
+import numpy as np
+import pytest
+
+from oracle import fem
+from opencmp_amd import _lib as L
+from opencmp_amd.mesh import unit_cube, unit_square
+
+pytestmark = pytest.mark.gpu
+
+
+def core():
+    from opencmp_amd import core as C
+    return C
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+# ------------------------------------------------------------------------------------------ load vectors
+
+POLY = {2: [0.3, -1.0, 2.0, 0.7, -0.4, 1.1], 3: [0.3, -1.0, 2.0, 0.5, 0.7, -0.4, 1.1, 0.2, -0.6, 0.9]}
+
+
+def poly(dim):
+    c = POLY[dim]
+    if dim == 2:
+        return lambda x, y: c[0] + c[1] * x + c[2] * y + c[3] * x * x + c[4] * x * y + c[5] * y * y
+    return lambda x, y, z: (c[0] + c[1] * x + c[2] * y + c[3] * z + c[4] * x * x + c[5] * y * y + c[6] * z * z +
+                            c[7] * x * y + c[8] * x * z + c[9] * y * z)
+
+
+# 2, 18 and 98 triangles, 6, 48 and 162 tetrahedra: one element tile of 16 and less, several with a rest
+@pytest.mark.parametrize('dim,n', [(2, 1), (2, 3), (2, 7), (3, 1), (3, 2), (3, 3)])
+@pytest.mark.parametrize('order', [1, 2, 3])
+def test_load_vector_tiles(gpu_ctx, dim, n, order):
+    """Volume loads of every order on tile edges, written and then accumulated, against the oracle's
+    quadrature (both rules exact for the data, so the difference is rounding: sums of at most 64 points and
+    24 elements, 1e-14 relative)."""
+    C = core()
+    hm = unit_square(n) if dim == 2 else unit_cube(n)
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.H1(order)])
+    f = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, POLY[dim]))])
+    f.Assemble()
+    cs = fem.Compound([fem.Space(fem.Topology(hm), 'H1', order)])
+    ref = fem.assemble_source(cs, 0, poly(dim))
+    assert rel(f.vec.cpu().numpy(), ref) < 1e-14
+    # nine terms: a second launch adds to the first's vector
+    f9 = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, POLY[dim]), coef=k + 1.0) for k in range(9)])
+    f9.Assemble()
+    assert rel(f9.vec.cpu().numpy(), 45.0 * ref) < 1e-14
+    f.Assemble()
+    assert rel(f.vec.cpu().numpy(), ref) < 1e-14
+
+
+def test_load_vector_blocks_and_facets(gpu_ctx):
+    """A compound space with terms on some blocks only, a boundary source on one marker, and no terms at
+    all: untouched blocks are zero."""
+    C = core()
+    hm = unit_square(5)
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.VectorH1(2), C.H1(1)])
+    t = fem.Topology(hm)
+    cs = fem.Compound([fem.Space(t, 'H1', 2, ncomp=2), fem.Space(t, 'H1', 1)])
+    right = hm.marker_mask('right')
+    f = C.LinearForm(fes, [C.Source(1, (L.FN_POLY2, POLY[2])), C.BndSource(0, right, fn=(L.FN_CONST, (2.0,)))])
+    f.Assemble()
+    ref = fem.assemble_source(cs, 0, [lambda x, y: 0 * x, poly(2)]) + \
+        fem.assemble_bnd_source(cs, 0, 2.0, right)
+    assert rel(f.vec.cpu().numpy(), ref) < 1e-14
+    only = C.LinearForm(fes, [C.BndSource(0, right, fn=(L.FN_CONST, (2.0,)))])
+    only.Assemble()
+    assert rel(only.vec.cpu().numpy(), fem.assemble_bnd_source(cs, 0, 2.0, right)) < 1e-14
+    none = C.LinearForm(fes, [])
+    none.vec.fill_(1.0)
+    none.Assemble()
+    assert float(none.vec.abs().max()) == 0.0
