@@ -78,3 +78,50 @@ def test_load_vector_blocks_and_facets(gpu_ctx):
     none.vec.fill_(1.0)
     none.Assemble()
     assert float(none.vec.abs().max()) == 0.0
+
+
+# ------------------------------------------------------------------------------------------ U-net
+
+
+@pytest.mark.parametrize('N', [4, 12, 16])
+def test_unet_tiles(gpu_ctx, N):
+    """Forward and parameter gradients where the 16-voxel tiles end inside a row: coarsest grids of 8, 64
+    and 125 voxels. The activations and the gradients of each layer are compared with the oracle's product
+    of the GPU's own stored inputs, so bf16 rounding does not travel: FP32 sums of at most 864 products
+    (1e-5 relative; an activation may differ by its own bf16 rounding, 2^-8, 4 % of them at most)."""
+    import torch
+    from opencmp_amd.learned import UNetPrecond
+    from oracle import unet as ou
+    from oracle.mlp import bf16_round
+    rng = np.random.default_rng(N)
+    p = (ou.init_params(N) + 0.05 * rng.standard_normal(ou.NPARAM)).astype(np.float32)
+    U = UNetPrecond(N, gpu_ctx, params=p)
+    n = [N + 1, N // 2 + 1, N // 4 + 1]
+    x = rng.standard_normal((4,) + (n[0],) * 3).astype(np.float32)
+    gy = rng.standard_normal((4,) + (n[0],) * 3).astype(np.float32)
+    g = U.grad(torch.tensor(x.reshape(4, -1), device='cuda'), torch.tensor(gy.reshape(4, -1), device='cuda'))
+    shapes = [(4, 0), (8, 0), (16, 1), (16, 1), (32, 2), (32, 2), (16, 1), (8, 0), (4, 0)]
+    a = [U.activation(l - 1).cpu().numpy().reshape((c,) + (n[lv],) * 3).astype(np.float64)
+         for l, (c, lv) in enumerate(shapes)]
+    q = {k: bf16_round(v).astype(np.float64) for k, v in ou.unpack(p).items()}
+    skip = {5: a[3], 6: a[1]}
+    for l, (name, kind, ci, co, s) in enumerate(ou.LAYERS):
+        W, b = q[name + '.W'], q[name + '.b']
+        z = ou.conv(a[l], W, b, s) if kind == 'c' else ou.tconv(a[l], W, b, a[l + 1].shape[1])
+        z = z + skip.get(l, 0.0)
+        if l < 7:
+            z = np.maximum(z, 0.0)
+            d = np.abs(a[l + 1] - z)
+            assert (d <= 2.0 ** -8 * np.abs(z) + 1e-5 * np.abs(z).max()).all(), name
+            r = bf16_round(z.astype(np.float32))
+            assert (a[l + 1] != r).mean() <= 0.04, name
+        else:
+            assert rel(a[8], z) < 1e-5
+    acts = {'x': a[0], **{f'a{l}': a[l + 1] for l in range(7)}}
+    _, gt = ou.backward(p, x, gy, bf16=True, acts=acts)
+    o = 0
+    g = g.cpu().numpy()
+    for name, kind, ci, co, s in ou.LAYERS:
+        for size in (ci * co * 27, co):
+            assert rel(g[o:o + size], gt[o:o + size]) < 1e-5, name
+            o += size
