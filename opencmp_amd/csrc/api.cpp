@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <array>
+#include <cstdlib>
 #include <cstring>
 #include <numeric>
 
@@ -410,53 +411,120 @@ void build_pattern(Matrix *A) {
   A->d_col.upload(A->col, st);
   A->d_val.alloc(A->nnz);
   OCMP_HIP(hipMemsetAsync(A->d_val.p, 0, A->nnz * sizeof(double), st));
-  build_row_blocks(A, A->rb64, SPMV_NNZB64);
+  build_row_blocks(A, A->rb, spmv_nnzb(A->nnz));
 }
 
 void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
-  // greedy: extend a block while its nonzeros fit in nnzb; a row longer than that is a block of
+  // greedy: extend a block while its nonzeros and rows fit; a row longer than that is a block of
   // its own (the kernel then loops over it in chunks and keeps global columns)
-  rb.rblk.clear();
-  rb.rblk.push_back(0);
+  const int64_t cap = nnzb - RB_ALIGN;
+  std::vector<int32_t> rblk;
+  rblk.push_back(0);
   int64_t start_nz = 0;
   for (int64_t r = 0; r < A->n; ++r) {
     const int64_t end_nz = A->row_ptr[r + 1];
-    if (end_nz - start_nz > nnzb && rb.rblk.back() != r) {
-      rb.rblk.push_back((int32_t)r);
+    if ((end_nz - start_nz > cap || r - rblk.back() >= RB_ROWS) && rblk.back() != r) {
+      rblk.push_back((int32_t)r);
       start_nz = A->row_ptr[r];
     }
   }
-  rb.rblk.push_back((int32_t)A->n);
-  rb.nrblk = (int64_t)rb.rblk.size() - 1;
-  rb.d_rblk.upload(rb.rblk, A->ctx->stream);
+  rblk.push_back((int32_t)A->n);
   // per block: its distinct columns, sorted, and for every nonzero the 16-bit position of its
-  // column in that list; the SpMV gathers x once per distinct column instead of once per nonzero
-  const int64_t nb = rb.nrblk;
-  std::vector<int32_t> nu(nb + 1, 0);
+  // column in that list; the SpMV gathers x once per distinct column instead of once per nonzero.
+  // A block with too many distinct columns is halved until none has.
+  int32_t cmax = -1;
+#pragma omp parallel for schedule(static) reduction(max : cmax)
+  for (int64_t j = 0; j < A->nnz; ++j) cmax = std::max(cmax, A->col[j]);
+  const int64_t ncol = (int64_t)cmax + 1;  // transfers between levels are not square
   std::vector<uint16_t> lcol(A->nnz);
-  std::vector<std::vector<int32_t>> ub(nb);
-#pragma omp parallel
-  {
-    std::vector<int32_t> buf;
-#pragma omp for schedule(dynamic, 256)
-    for (int64_t b = 0; b < nb; ++b) {
-      const int64_t j0 = A->row_ptr[rb.rblk[b]], j1 = A->row_ptr[rb.rblk[b + 1]];
-      if (j1 - j0 > nnzb) continue;
-      buf.assign(A->col.begin() + j0, A->col.begin() + j1);
-      std::sort(buf.begin(), buf.end());
-      buf.erase(std::unique(buf.begin(), buf.end()), buf.end());
-      for (int64_t j = j0; j < j1; ++j)
-        lcol[j] = (uint16_t)(std::lower_bound(buf.begin(), buf.end(), A->col[j]) - buf.begin());
-      nu[b + 1] = (int32_t)buf.size();
-      ub[b] = buf;
+  std::vector<std::vector<int32_t>> ub;
+  std::vector<uint8_t> done;  // blocks whose list is built
+  for (;;) {
+    const int64_t nb = (int64_t)rblk.size() - 1;
+    if (done.empty()) {
+      ub.assign(nb, {});
+      done.assign(nb, 0);
     }
+    std::vector<uint8_t> over(nb, 0);
+    bool any = false;
+    // per thread and column: the last block of the thread that has it, and its position in that
+    // block's list. Zeroed lazily by the system: a thread's blocks are consecutive and touch few pages.
+    struct Col {
+      int32_t blk, pos;
+    };
+    std::vector<std::unique_ptr<Col, void (*)(void *)>> seen;
+    for (int t = 0; t < omp_get_max_threads(); ++t) {
+      seen.emplace_back((Col *)std::calloc(std::max<int64_t>(ncol, 1), sizeof(Col)), std::free);
+      if (!seen.back()) throw std::bad_alloc();
+    }
+#pragma omp parallel
+    {
+      Col *const col_of = seen[omp_get_thread_num()].get();
+      std::vector<int32_t> buf;
+      int32_t id = 0;
+#pragma omp for schedule(static) reduction(|| : any)
+      for (int64_t b = 0; b < nb; ++b) {
+        if (done[b]) continue;
+        done[b] = 1;
+        const int64_t j0 = A->row_ptr[rblk[b]], j1 = A->row_ptr[rblk[b + 1]];
+        if (j1 - j0 > cap) continue;
+        ++id;
+        buf.clear();
+        for (int64_t j = j0; j < j1; ++j) {
+          Col &c = col_of[A->col[j]];
+          if (c.blk != id) {
+            c.blk = id;
+            buf.push_back(A->col[j]);
+          }
+        }
+        if ((int64_t)buf.size() > RB_XCAP) {
+          if (rblk[b + 1] - rblk[b] > 1) {
+            over[b] = 1;
+            any = true;
+          }
+          continue;
+        }
+        std::sort(buf.begin(), buf.end());
+        for (size_t i = 0; i < buf.size(); ++i) col_of[buf[i]].pos = (int32_t)i;
+        for (int64_t j = j0; j < j1; ++j) lcol[j] = (uint16_t)col_of[A->col[j]].pos;
+        ub[b] = buf;
+      }
+    }
+    if (!any) break;
+    std::vector<int32_t> nr;
+    std::vector<std::vector<int32_t>> nu2;
+    std::vector<uint8_t> nd;
+    for (int64_t b = 0; b < nb; ++b) {
+      nr.push_back(rblk[b]);
+      nu2.push_back(std::move(ub[b]));
+      nd.push_back(!over[b]);
+      if (over[b]) {
+        nr.push_back((rblk[b] + rblk[b + 1]) / 2);
+        nu2.emplace_back();
+        nd.push_back(0);
+      }
+    }
+    nr.push_back((int32_t)A->n);
+    rblk.swap(nr);
+    ub.swap(nu2);
+    done.swap(nd);
   }
-  for (int64_t b = 0; b < nb; ++b) nu[b + 1] += nu[b];
+  const int64_t nb = rb.nrblk = (int64_t)rblk.size() - 1;
+  std::vector<int32_t> nu(nb + 1, 0);
+  for (int64_t b = 0; b < nb; ++b) nu[b + 1] = nu[b] + (int32_t)ub[b].size();
   std::vector<int32_t> ucol(nu[nb]);
+  std::vector<RbDesc> desc(nb);
 #pragma omp parallel for schedule(static)
-  for (int64_t b = 0; b < nb; ++b) std::copy(ub[b].begin(), ub[b].end(), ucol.begin() + nu[b]);
+  for (int64_t b = 0; b < nb; ++b) {
+    std::copy(ub[b].begin(), ub[b].end(), ucol.begin() + nu[b]);
+    const int32_t r0 = rblk[b], r1 = rblk[b + 1], nz = A->row_ptr[r1] - A->row_ptr[r0];
+    int kind = nz > 0 && ub[b].empty() ? RB_LONG_ROW : RB_PLAIN;
+    for (int32_t r = r0; r < r1; ++r)
+      if (A->row_ptr[r] == A->row_ptr[r + 1]) kind = RB_HAS_EMPTY;
+    desc[b] = RbDesc{r0, r1 - r0, A->row_ptr[r0], nz, nu[b], nu[b + 1] - nu[b], kind, 0};
+  }
   rb.nucol = nu[nb];
-  rb.d_ubase.upload(nu, A->ctx->stream);
+  rb.d_desc.upload(desc, A->ctx->stream);
   rb.d_ucol.upload(ucol, A->ctx->stream);
   rb.d_lcol.upload(lcol, A->ctx->stream);
   rb.nnzb = nnzb;
@@ -534,7 +602,7 @@ void build_solver_operator(Matrix *A) {
   M->d_src.upload(src.empty() ? std::vector<int32_t>(1, 0) : src, st);
   M->d_rowmap.upload(order, st);
   M->d_val.alloc(std::max<int64_t>(M->nnz, 1));
-  build_row_blocks(M, M->rb64, SPMV_NNZB64);
+  build_row_blocks(M, M->rb, spmv_nnzb(M->nnz));
   M->assembled = true;
   OCMP_HIP(hipStreamSynchronize(st));
   delete A->op;
@@ -554,10 +622,6 @@ void ensure_diag_slots(Matrix *A) {
   }
   A->d_dslot.upload(d, A->ctx->stream);
   OCMP_HIP(hipStreamSynchronize(A->ctx->stream));
-}
-
-void ensure_row_blocks32(Matrix *A) {
-  if (!A->rb32.nnzb) build_row_blocks(A, A->rb32, SPMV_NNZB32);
 }
 
 // the dof range [s0, s1) of the Schur blocks, which must be adjacent
@@ -634,7 +698,7 @@ void build_schur_matrix(Precond *P) {
   S->d_row_ptr.upload(S->row_ptr, st);
   S->d_col.upload(S->col, st);
   S->d_val.alloc(nnz);
-  build_row_blocks(S, S->rb64, SPMV_NNZB64);
+  build_row_blocks(S, S->rb, SPMV_NNZB);
   build_row_blocks(S, P->srb, SCG_NNZB);
   S->assembled = true;
   P->d_sseg.upload(seg, st);
@@ -746,7 +810,7 @@ Matrix *amg_matrix(Matrix *like, const HCsr &h) {
   M->d_row_ptr.upload(M->row_ptr, st);
   M->d_col.upload(M->col, st);
   M->d_val.alloc(std::max<int64_t>(M->nnz, 1));
-  build_row_blocks(M, M->rb64, SPMV_NNZB64);
+  build_row_blocks(M, M->rb, SPMV_NNZB);
   M->assembled = true;
   return M;
 }
@@ -1167,7 +1231,7 @@ void build_velocity_blocks(Precond *P) {
     M->d_row_ptr.upload(M->row_ptr, st);
     M->d_col.upload(M->col, st);
     M->d_val.alloc(M->nnz);
-    build_row_blocks(M, M->rb64, SPMV_NNZB64);
+    build_row_blocks(M, M->rb, spmv_nnzb(M->nnz));
     M->assembled = true;
     return M;
   };

@@ -33,7 +33,10 @@ void set_error(const std::string &msg);
     if (!(cond)) throw ::ocmp::Error(OCMP_ERR_ARG, std::string(msg));   \
   } while (0)
 
-// Device buffer owned by the library.
+// Device buffer owned by the library, with DBUF_SLACK bytes behind its last element: the CSR kernels
+// load a thread's run of nonzeros in 16-byte pieces, which may end past the array's end (the
+// surplus is read and dropped).
+constexpr size_t DBUF_SLACK = 128;
 template <class T>
 struct DBuf {
   T *p = nullptr;
@@ -45,7 +48,7 @@ struct DBuf {
   void alloc(size_t count) {
     if (count == n && p) return;
     release();
-    if (count) OCMP_HIP(hipMalloc((void **)&p, count * sizeof(T)));
+    if (count) OCMP_HIP(hipMalloc((void **)&p, count * sizeof(T) + DBUF_SLACK));
     n = count;
   }
   void release() {
@@ -226,13 +229,23 @@ struct bf16s {
   }
 };
 
-// Rows grouped into blocks of at most nnzb nonzeros (block b = rows [rblk[b], rblk[b+1])), the
-// distinct columns of each block (ucol[ubase[b] .. ubase[b+1]), sorted) and every nonzero's
-// 16-bit position in its block's list.
+// Rows grouped into blocks of at most nnzb - RB_ALIGN nonzeros, RB_ROWS rows and RB_XCAP distinct
+// columns (or a single row that exceeds them), the distinct columns of each block (ucol[u0 .. u0 + nu),
+// sorted) and every nonzero's 16-bit position in its block's list. The kernels read a block's nonzeros from the multiple of RB_ALIGN
+// at or below its first one, so that they are aligned: the block still fits in nnzb.
+constexpr int RB_ALIGN = 8, RB_ROWS = 512, RB_XCAP = 2048;
+enum { RB_PLAIN = 0, RB_HAS_EMPTY = 1 /* some row has no nonzeros */, RB_LONG_ROW = 2 };
+struct RbDesc {
+  int32_t r0, nrows;   // rows
+  int32_t j0, nz;      // nonzeros
+  int32_t u0, nu;      // distinct columns
+  int32_t kind;        // RB_*
+  int32_t pad;
+};
 struct RowBlocks {
   int nnzb = 0;  // 0: not built
-  std::vector<int32_t> rblk;
-  DBuf<int32_t> d_rblk, d_ubase, d_ucol;
+  DBuf<RbDesc> d_desc;
+  DBuf<int32_t> d_ucol;
   DBuf<uint16_t> d_lcol;
   int64_t nrblk = 0, nucol = 0;
 };
@@ -277,9 +290,7 @@ struct Matrix {
   DBuf<int8_t> d_dg_pos;             // nel*(dim+2): pos of diag block, then of each facet neighbour (-1 none)
   DBuf<int32_t> d_dg_bcol;           // nel*4 block columns (-1 padded), sorted
   int dg_nb = 0;                     // local dofs per element (block size)
-  // LDS-staged SpMV row blocks: FP64 values use blocks of SPMV_NNZB64 nonzeros, FP32 values
-  // (built with the FP32 copy) blocks of SPMV_NNZB32
-  RowBlocks rb64, rb32;
+  RowBlocks rb;  // row blocks of the LDS-staged SpMV, of spmv_nnzb(nnz) nonzeros
   bool assembled = false;
   // mixed precision copy
   DBuf<float> d_val32;
@@ -463,17 +474,17 @@ void build_h1_schedule(Matrix *A);
 void build_h1_gather(Matrix *A);
 void build_colouring(Space &s);
 void build_pattern(Matrix *A);
-// nonzeros per row block of the LDS-staged SpMV (LDS: 16 KB per block in both precisions;
-// measured on H1 P3, 7.2M dofs: FP64 1.01 ms at 2048 against 1.04 at 3072 and 1.20 at 4096,
-// FP32 0.69 ms at 4096 against 0.83 at 2048 and 0.85 at 8192)
-constexpr int SPMV_NNZB64 = 2048;
-constexpr int SPMV_NNZB32 = 4096;
+// nonzeros per row block of the LDS-staged SpMV: large blocks where there are enough of them for
+// several a CU (62M FP64 nonzeros: 157 us against 169 with small ones), small ones below, where one
+// block's chain of loads and sums is the launch's time
+constexpr int SPMV_NNZB = 2048, SPMV_NNZB_LARGE = 4096;
+constexpr int64_t SPMV_LARGE_NNZ = (int64_t)4 << 20;
+inline int spmv_nnzb(int64_t nnz) { return nnz >= SPMV_LARGE_NNZ ? SPMV_NNZB_LARGE : SPMV_NNZB; }
 // the fused Schur PCG iteration: row blocks of S of this many nonzeros, SCG_NT threads a block
 constexpr int SCG_NNZB = 4096;
 constexpr int SCG_NT = 512;
 void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb);
 void build_solver_operator(Matrix *A);
-void ensure_row_blocks32(Matrix *A);
 // the pattern of a Schur preconditioner's S = C + B diag(A)^{-1} B^T and the per-row Schur
 // column ranges of A (host, once per preconditioner)
 void build_schur_matrix(Precond *P);

@@ -137,13 +137,18 @@ __global__ void k_reduce(const double *__restrict__ part, int nparts, double *__
 
 // ------------------------------------------------------------------ CSR SpMV
 
-// LDS-staged CSR SpMV. Block b owns rows [rblk[b], rblk[b+1]) whose nonzeros form one
-// contiguous range of at most NNZB entries. The block first gathers x at its distinct
-// columns (ucol, sorted: neighbouring lanes read neighbouring entries) into LDS; every thread
-// then loads NNZB/256 (16-bit local column, value) pairs with fully coalesced loads and stages the
-// products in LDS; rows are summed from LDS by 4 lanes each. The rows of a finite-element block
-// share most of their columns, so the x gathers (the texture-unit bound part of a plain CSR
-// SpMV) drop several-fold, and the 16-bit local columns save 2 bytes per nonzero.
+// LDS-staged CSR SpMV. A block owns consecutive rows whose nonzeros form one contiguous range of less
+// than NNZB entries. It first gathers x at its distinct columns (ucol, sorted: neighbouring lanes
+// read neighbouring entries) into LDS; every thread then takes NNZB / NT consecutive nonzeros as
+// 16-byte loads of values and 16-bit local columns, and adds its products in a register, leaving a
+// partial sum in LDS where a row ends and at the end of its run; one thread per row adds the few
+// partial sums of its row. The rows of a finite-element block share most of their columns, so the
+// x gathers (the texture-unit bound part of a plain CSR SpMV) drop several-fold, and the 16-bit
+// local columns save 2 bytes per nonzero. Against products staged in LDS and summed by four lanes
+// per row from there (strided 4-byte and 2-byte loads, two more LDS accesses per nonzero): FP32
+// operator of the INS channel, 40M nonzeros, 68 -> 50 us (5.0 TB/s of its 252 MB); 3D P3 with 43M
+// nonzeros FP32 93 -> 66 us, FP64 133 -> 123 us; 4,225 rows 7.3 -> 5.2 us (fewer dependent loads:
+// one descriptor per block).
 //
 // mode 0: y = A x
 // mode 1: y = mask*(b - A x), partial sum y^2 (y == nullptr: the partial sum only)
@@ -181,134 +186,187 @@ __device__ __forceinline__ void spmv_epilogue(int mode, int64_t r, double s, XT 
   }
 }
 
-// One row block of a CSR product: the x values at the block's distinct columns (xl(c) loads the
-// value at column c, xs(c, v) then scales it) are staged in LDS, each thread forms its share of the products, and 4 lanes
-// per row sum them in a fixed order; ef(r, s) receives each row's sum. The LDS buffer holds first
-// the staged x values, then (after every thread has read its operands) the products, so the
-// kernel's LDS is exactly NNZB values (a power of two: whole blocks per CU).
-template <typename VT, typename XT, int NNZB, typename XL, typename XS, typename EF>
-__device__ __forceinline__ void csr_row_block(int lb, const int32_t *__restrict__ rblk, const int32_t *__restrict__ rp,
-                                              const int32_t *__restrict__ col, const int32_t *__restrict__ ubase,
-                                              const int32_t *__restrict__ ucol, const uint16_t *__restrict__ lcol,
-                                              const VT *__restrict__ val, double *lds, XL xl, XS xsc, EF ef) {
-  constexpr int SPMV_PER_THREAD = NNZB / NTHR;
-  XT *xs = reinterpret_cast<XT *>(lds);
-  XT *prod = xs;
-  const int32_t r0 = rblk[lb], r1 = rblk[lb + 1];
-  const int32_t j0 = rp[r0], j1 = rp[r1];
-  const int nz = j1 - j0;
-  const int nrows = r1 - r0;
-  if (nz <= NNZB) {
-    // rows of the first pass: fetch their bounds early so the loads overlap the staging
-    const int ri0 = threadIdx.x >> 2, q = threadIdx.x & 3;
-    int a0 = 0, e0 = 0;
-    if (ri0 < nrows) {
-      a0 = rp[r0 + ri0] - j0;
-      e0 = rp[r0 + ri0 + 1] - j0;
-    }
-    int li[SPMV_PER_THREAD];
-    VT vv[SPMV_PER_THREAD];
+// a CSR matrix with its row blocks, as one kernel argument
+template <typename T>
+struct RbCsr {
+  int64_t nrblk;
+  const RbDesc *desc;
+  const int32_t *rp, *col, *ucol;
+  const uint16_t *lcol;
+  const T *val;
+};
+template <typename T>
+static RbCsr<T> rb_csr(const Matrix *A, const RowBlocks &rb, const T *val) {
+  return {rb.nrblk, rb.d_desc.p, A->d_row_ptr.p, A->d_col.p, rb.d_ucol.p, rb.d_lcol.p, val};
+}
+
+// LDS of one row block
+template <typename XT, int NNZB, int NT>
+struct RbLds {
+  XT xs[RB_XCAP];            // x at the distinct columns
+  XT fin[RB_ROWS];           // per row: the sum of its last run's part
+  XT car[NT];                // per run: the sum after its last row end
+  unsigned ends[NT];         // per run: bit k set where its k-th nonzero ends a row
+  uint16_t row[NT];          // per run: the row of its first nonzero
+  double red[2 * NT / 64];
+};
+
+// N consecutive elements from a 16-byte aligned address
+template <int N, typename T>
+__device__ __forceinline__ void load_run(const T *__restrict__ p, T (&v)[N]) {
+  static_assert(N * sizeof(T) % 16 == 0, "whole 16-byte loads");
+  union {
+    uint4 q[N * sizeof(T) / 16];
+    T t[N];
+  } u;
 #pragma unroll
-    for (int k = 0; k < SPMV_PER_THREAD; ++k) {
-      const int t = threadIdx.x + k * NTHR;
-      li[k] = -1;
-      vv[k] = (VT)0;
-      if (t < nz) {
-        li[k] = lcol[j0 + t];
-        vv[k] = val[j0 + t];
+  for (int i = 0; i < (int)(N * sizeof(T) / 16); ++i) u.q[i] = reinterpret_cast<const uint4 *>(p)[i];
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = u.t[i];
+}
+
+// One row block of a CSR product: xl(c) gives the (scaled) x value at column c, ef(r, s) receives each
+// row's sum, always in the same order of additions. Sums in the vector type (FP32 products in FP32,
+// FP64 in FP64).
+template <typename VT, typename XT, int NNZB, int NT, typename XL, typename EF>
+__device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, RbLds<XT, NNZB, NT> &S, XL xl, EF ef) {
+  constexpr int PER = NNZB / NT;
+  static_assert(PER % RB_ALIGN == 0 && PER <= 32, "runs are aligned and fit the mask");
+  constexpr int RPT = RB_ROWS / NT;  // rows per thread
+  const RbDesc D = M.desc[lb];
+  const int tid = threadIdx.x;
+  if (D.kind == RB_LONG_ROW) {
+    double s = 0.0;
+    for (int t = tid; t < D.nz; t += NT) {
+      const int32_t c = M.col[D.j0 + t];
+      s += (double)((XT)M.val[D.j0 + t] * xl(c));
+    }
+    s = block_sum(s, S.red);
+    if (tid == 0) ef((int64_t)D.r0, s);
+    return;
+  }
+  const int jb = D.j0 & ~(RB_ALIGN - 1);  // where the runs start
+  const int d = D.j0 - jb, end = d + D.nz;
+  const int p0 = tid * PER;
+  VT v[PER];
+  uint16_t li[PER];
+  const bool active = p0 < end;
+  if (active) {
+    load_run<PER>(M.val + jb + p0, v);
+    load_run<PER>(M.lcol + jb + p0, li);
+  }
+  int ra[RPT], re[RPT];
+#pragma unroll
+  for (int k = 0; k < RPT; ++k) {
+    const int ri = min(tid + k * NT, D.nrows - 1);
+    ra[k] = M.rp[D.r0 + ri] - jb;
+    re[k] = M.rp[D.r0 + ri + 1] - jb;
+  }
+  S.ends[tid] = 0u;
+  __syncthreads();
+  // x at the distinct columns (indices past nu are clamped so that a round's gathers are unconditional)
+  for (int base = 0; base < D.nu; base += 4 * NT) {
+    int32_t c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = M.ucol[D.u0 + min(base + k * NT + tid, D.nu - 1)];
+    XT x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = xl(c[k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int t = base + k * NT + tid;
+      if (t < D.nu) S.xs[t] = x[k];
+    }
+  }
+  if (D.kind == RB_PLAIN) {
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int ri = tid + k * NT;
+      if (ri < D.nrows) {
+        atomicOr(&S.ends[(re[k] - 1) / PER], 1u << ((re[k] - 1) % PER));
+        // the runs whose first nonzero is in this row (row 0 also has the run that starts before it)
+        for (int t = ri == 0 ? 0 : (ra[k] + PER - 1) / PER; t * PER < re[k]; ++t) S.row[t] = (uint16_t)ri;
       }
     }
-    // x at the block's distinct columns (nu >= 1 since nz >= 1; indices past nu are clamped
-    // so both gathers of a round are unconditional)
-    const int u0 = ubase[lb], nu = ubase[lb + 1] - u0;
-    for (int base = 0; base < nu; base += 2 * NTHR) {
-      const int t0 = base + threadIdx.x, t1 = t0 + NTHR;
-      const int32_t c0 = ucol[u0 + min(t0, nu - 1)], c1 = ucol[u0 + min(t1, nu - 1)];
-      XT x0 = xl(c0), x1 = xl(c1);
-      x0 = xsc(c0, x0);
-      x1 = xsc(c1, x1);
-      if (t0 < nu) xs[t0] = x0;
-      if (t1 < nu) xs[t1] = x1;
-    }
     __syncthreads();
-    XT pv[SPMV_PER_THREAD];
+    if (active) {
+      if (p0 < d || p0 + PER > end) {  // a run with entries of a neighbouring block
 #pragma unroll
-    for (int k = 0; k < SPMV_PER_THREAD; ++k) pv[k] = li[k] >= 0 ? (XT)vv[k] * xs[li[k]] : (XT)0;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < SPMV_PER_THREAD; ++k)
-      if (li[k] >= 0) prod[threadIdx.x + k * NTHR] = pv[k];
-    __syncthreads();
-    for (int base = 0; base < nrows; base += NTHR / 4) {
-      const int ri = base + ri0;
-      int a = a0, e = e0;
-      if (base > 0 && ri < nrows) {
-        a = rp[r0 + ri] - j0;
-        e = rp[r0 + ri + 1] - j0;
+        for (int k = 0; k < PER; ++k)
+          if (p0 + k < d || p0 + k >= end) {
+            v[k] = (VT)0;
+            li[k] = 0;
+          }
       }
-      // partial row sums in the vector type (FP32 products summed in FP32, FP64 in FP64)
+      XT xv[PER];
+#pragma unroll
+      for (int k = 0; k < PER; ++k) xv[k] = S.xs[li[k]];
+      const unsigned m = S.ends[tid];
+      int row = S.row[tid];
       XT s = (XT)0;
-      if (ri < nrows)
-        for (int t = a + q; t < e; t += 4) s += prod[t];
-      s += __shfl_xor(s, 1, 4);
-      s += __shfl_xor(s, 2, 4);
-      if (ri < nrows && q == 0) ef((int64_t)(r0 + ri), (double)s);
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        s += (XT)v[k] * xv[k];
+        if (m >> k & 1u) {
+          S.fin[row++] = s;
+          s = (XT)0;
+        }
+      }
+      S.car[tid] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int ri = tid + k * NT;
+      if (ri < D.nrows) {
+        XT s = (XT)0;
+        const int tb = (re[k] - 1) / PER;
+        for (int t = ra[k] / PER; t < tb; ++t) s += S.car[t];
+        s += S.fin[ri];
+        ef((int64_t)(D.r0 + ri), (double)s);
+      }
     }
   } else {
-    // a single row longer than the staging buffer
-    double s = 0.0;
-    for (int t = threadIdx.x; t < nz; t += NTHR) {
-      const int32_t c = col[j0 + t];
-      s += (double)((XT)val[j0 + t] * xsc(c, xl(c)));
+    // rows without nonzeros among them (left-out rows of a multigrid level): a thread per row
+    __syncthreads();
+    for (int ri = tid; ri < D.nrows; ri += NT) {
+      XT s = (XT)0;
+      for (int32_t j = M.rp[D.r0 + ri]; j < M.rp[D.r0 + ri + 1]; ++j) s += (XT)M.val[j] * S.xs[M.lcol[j]];
+      ef((int64_t)(D.r0 + ri), (double)s);
     }
-    s = block_sum(s, lds);
-    if (threadIdx.x == 0) ef((int64_t)r0, s);
   }
 }
 
-template <typename VT, typename XT, int NNZB>
-__global__ void __launch_bounds__(NTHR) k_spmv_csr(int64_t nrblk, const int32_t *__restrict__ rblk,
-                                                   const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
-                                                   const int32_t *__restrict__ ubase,
-                                                   const int32_t *__restrict__ ucol,
-                                                   const uint16_t *__restrict__ lcol,
-                                                   const VT *__restrict__ val, const XT *__restrict__ x,
-                                                   XT *__restrict__ y, const double *__restrict__ b,
-                                                   const uint8_t *__restrict__ mask, const XT *__restrict__ cs,
-                                                   const double *__restrict__ sx, int mode,
+template <typename VT, typename XT, int NNZB, int NT>
+__global__ void __launch_bounds__(NT) k_spmv_csr(RbCsr<VT> M, const XT *__restrict__ x, XT *__restrict__ y,
+                                                   const double *__restrict__ b, const uint8_t *__restrict__ mask,
+                                                   const XT *__restrict__ cs, const double *__restrict__ sx, int mode,
                                                    double *__restrict__ part, XT dsh, const XT *__restrict__ xp,
                                                    XT csh, const int *__restrict__ skip,
                                                    const int32_t *__restrict__ rowmap) {
   if (skip && *skip) return;  // a converged inner solve: the rest of its fixed launch sequence is empty
-  __shared__ double lds[NNZB * sizeof(XT) / sizeof(double)];
+  __shared__ RbLds<XT, NNZB, NT> lds;
   const int lb = xcd_block();
   double acc = 0.0;
   const XT scale = (mode == 3 && sx) ? (XT)sx[0] : (XT)1;
-  if (lb < nrblk)
-    csr_row_block<VT, XT, NNZB>(
-        lb, rblk, rp, col, ubase, ucol, lcol, val, lds,
-        [&](int32_t c) { return x[c]; },
-        [&](int32_t c, XT v) { return (mode >= 3 && cs) ? v * cs[c] : v; },
+  if (lb < M.nrblk)
+    csr_row_block<VT, XT, NNZB, NT>(
+        M, lb, lds,
+        [&](int32_t c) { return (mode >= 3 && cs) ? x[c] * cs[c] : x[c]; },
         [&](int64_t r, double s) {
           // a reordered operator's row r is row rowmap[r] of the vectors
           spmv_epilogue<VT, XT>(mode, rowmap ? (int64_t)rowmap[r] : r, s, y, x, b, mask, scale, acc, dsh, xp, csh);
         });
   if (part) {
-    __syncthreads();  // the block-sum scratch aliases the products
-    acc = block_sum(acc, lds);
+    __syncthreads();
+    acc = block_sum(acc, lds.red);
     if (threadIdx.x == 0) part[lb] = acc;
   }
 }
 
-// FP32 values and vectors use the larger row blocks (same 16 KB of LDS)
-template <typename VT, typename XT>
-static const RowBlocks &row_blocks(const Matrix *A) {
-  return (sizeof(VT) == 4 && sizeof(XT) == 4 && A->rb32.nnzb) ? A->rb32 : A->rb64;
-}
-
 template <typename VT, typename XT>
 static int spmv_grid(Matrix *A) {
-  int64_t g = std::max<int64_t>(row_blocks<VT, XT>(A).nrblk, NXCD);
+  int64_t g = std::max<int64_t>(A->rb.nrblk, NXCD);
   g = (g + NXCD - 1) / NXCD * NXCD;
   return (int)g;
 }
@@ -318,24 +376,23 @@ template <typename VT, typename XT>
 static void spmv_dispatch(Matrix *A, const VT *val, const XT *x, XT *y, const double *b, const uint8_t *mask,
                           const XT *cs, const double *sx, int mode, double *part, int grid, hipStream_t st,
                           XT dsh = (XT)0, const XT *xp = nullptr, XT csh = (XT)0, const int *skip = nullptr) {
-  const RowBlocks &rb = row_blocks<VT, XT>(A);
   OCMP_REQUIRE((grid == spmv_grid<VT, XT>(A)), "SpMV grid does not match the row blocks");
-  if (rb.nnzb == SPMV_NNZB32)
-    k_spmv_csr<VT, XT, SPMV_NNZB32><<<grid, NTHR, 0, st>>>(rb.nrblk, rb.d_rblk.p, A->d_row_ptr.p, A->d_col.p,
-                                                          rb.d_ubase.p, rb.d_ucol.p, rb.d_lcol.p, val, x, y, b,
-                                                          mask, cs, sx, mode, part, dsh, xp, csh, skip,
-                                                          A->d_rowmap.p);
+  const RbCsr<VT> M = rb_csr<VT>(A, A->rb, val);
+  // runs of 16 FP32 or 8 FP64 nonzeros a thread in the large blocks (64 bytes of values; on 62M FP64 nonzeros
+  // 157 us, with runs of 16 181), of 8 in the small ones
+  constexpr int NTL = sizeof(VT) == 8 ? 512 : NTHR;
+  if (A->rb.nnzb == SPMV_NNZB_LARGE)
+    k_spmv_csr<VT, XT, SPMV_NNZB_LARGE, NTL><<<grid, NTL, 0, st>>>(M, x, y, b, mask, cs, sx, mode, part, dsh, xp, csh,
+                                                                   skip, A->d_rowmap.p);
   else
-    k_spmv_csr<VT, XT, SPMV_NNZB64><<<grid, NTHR, 0, st>>>(rb.nrblk, rb.d_rblk.p, A->d_row_ptr.p, A->d_col.p,
-                                                          rb.d_ubase.p, rb.d_ucol.p, rb.d_lcol.p, val, x, y, b,
-                                                          mask, cs, sx, mode, part, dsh, xp, csh, skip,
-                                                          A->d_rowmap.p);
+    k_spmv_csr<VT, XT, SPMV_NNZB, NTHR><<<grid, NTHR, 0, st>>>(M, x, y, b, mask, cs, sx, mode, part, dsh, xp, csh,
+                                                               skip, A->d_rowmap.p);
 }
 
 // algorithmic bytes of one CSR SpMV: values + 16-bit local columns + the blocks' distinct
 // columns + row pointers + x once + y once
 static double csr_bytes(const Matrix *A, int wv, int wx) {
-  const RowBlocks &rb = (wv == 4 && wx == 4 && A->rb32.nnzb) ? A->rb32 : A->rb64;
+  const RowBlocks &rb = A->rb;
   return (double)A->nnz * (wv + 2) + 4.0 * rb.nucol + 4.0 * (A->n + 1) + 2.0 * A->n * wx +
          (A->d_rowmap.p ? 4.0 * A->n : 0.0);
 }
@@ -1527,20 +1584,6 @@ __global__ void k_amg_wvals(int64_t nw, const int32_t *__restrict__ wrow, const 
   if (wval32) wval32[e] = (float)v;
 }
 
-// a CSR matrix with its row blocks, as one kernel argument
-template <typename T>
-struct RbCsr {
-  int64_t nrblk;
-  const int32_t *rblk, *rp, *col, *ubase, *ucol;
-  const uint16_t *lcol;
-  const T *val;
-};
-template <typename T>
-static RbCsr<T> rb_csr(const Matrix *A, const T *val) {
-  const RowBlocks &rb = A->rb64;
-  return {rb.nrblk, rb.d_rblk.p, A->d_row_ptr.p, A->d_col.p, rb.d_ubase.p, rb.d_ucol.p, rb.d_lcol.p, val};
-}
-
 // The descending half of a V(1,1) level with the input b = g u (g = -sig[0], or 1 without sig):
 // the first ga logical blocks form z = w D^-1 (2 b - w A D^-1 b) (the iterate after damped-Jacobi
 // pre-smoothing from zero and post-smoothing without the coarse correction), the rest the
@@ -1561,7 +1604,7 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
                                                    const T *__restrict__ dinv, const double *__restrict__ sig,
                                                    T w, T *__restrict__ z, T *__restrict__ bc, T *__restrict__ bout,
                                                    JacRows<T> J, const int *__restrict__ skip) {
-  __shared__ double lds[NNZB * sizeof(T) / sizeof(double)];
+  __shared__ RbLds<T, NNZB, NTHR> lds;
   if (skip && *skip) return;  // a converged FGMRES cycle: its remaining launches are empty
   const int lb = xcd_block();
   const double g = sig ? -sig[0] : 1.0;
@@ -1574,9 +1617,8 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
   }
   if (lb < ga) {
     if (lb >= A.nrblk) return;
-    csr_row_block<T, T, NNZB>(
-        lb, A.rblk, A.rp, A.col, A.ubase, A.ucol, A.lcol, A.val, lds, [&](int32_t c) { return u[c]; },
-        [&](int32_t c, T v) { return v * dinv[c]; },
+    csr_row_block<T, T, NNZB, NTHR>(
+        A, lb, lds, [&](int32_t c) { return u[c] * dinv[c]; },
         [&](int64_t r, double s) {
           const double b = g * (double)u[r];
           z[r] = (T)((double)w * (double)dinv[r] * (2.0 * b - (double)w * g * s));
@@ -1585,9 +1627,8 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
   } else {
     const int wb = lb - ga;
     if (wb >= Wt.nrblk) return;
-    csr_row_block<T, T, NNZB>(
-        wb, Wt.rblk, Wt.rp, Wt.col, Wt.ubase, Wt.ucol, Wt.lcol, Wt.val, lds, [&](int32_t c) { return u[c]; },
-        [&](int32_t, T v) { return v; }, [&](int64_t r, double s) { bc[r] = (T)(g * s); });
+    csr_row_block<T, T, NNZB, NTHR>(
+        Wt, wb, lds, [&](int32_t c) { return u[c]; }, [&](int64_t r, double s) { bc[r] = (T)(g * s); });
   }
 }
 
@@ -1816,8 +1857,8 @@ static void amg_vcycle(Amg &M, size_t l, const T *u, const double *sig, T *x, T 
   T *z = vecs(L) + 2 * n;
   T *bc = vecs(C), *xc = vecs(C) + C.A->n;
   const int ga = spmv_grid<double, double>(L.A), gw = spmv_grid<double, double>(L.Wt);
-  const RbCsr<T> a = rb_csr<T>(L.A, vals(L.A)), wt = rb_csr<T>(L.Wt, vals(L.Wt));
-  k_amg_down<T, SPMV_NNZB64><<<ga + gw + J.nblk, NTHR, 0, st>>>(ga, a, wt, u, dinv, sig, (T)AMG_SMOOTH, z, bc, bout,
+  const RbCsr<T> a = rb_csr<T>(L.A, L.A->rb, vals(L.A)), wt = rb_csr<T>(L.Wt, L.Wt->rb, vals(L.Wt));
+  k_amg_down<T, SPMV_NNZB><<<ga + gw + J.nblk, NTHR, 0, st>>>(ga, a, wt, u, dinv, sig, (T)AMG_SMOOTH, z, bc, bout,
                                                                  J, skip);
   amg_vcycle<T>(M, l + 1, bc, nullptr, xc, nullptr, st, JacRows<T>{0, 0, nullptr, nullptr, nullptr, nullptr}, skip);
   spmv_dispatch<T, T>(L.W, vals(L.W), xc, x, nullptr, nullptr, nullptr, nullptr, 6, nullptr, spmv_grid<T, T>(L.W), st,
@@ -2040,7 +2081,6 @@ void precond_update(Precond *P) {
         refresh_val32(A, st);
       else
         A->d_val32.alloc(A->nnz);
-      ensure_row_blocks32(A);
     }
   } else {
     const Mesh &m = *A->space->mesh;
@@ -3146,18 +3186,13 @@ __device__ __forceinline__ ScgNext<T> scg_next(const T *__restrict__ rin, const 
 
 template <typename T, typename VT, int NNZB, int NT>
 __global__ void __launch_bounds__(NT) k_scg_fused(
-    int64_t nrblk, const int32_t *__restrict__ rblk, const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
-    const int32_t *__restrict__ ubase, const int32_t *__restrict__ ucol, const uint16_t *__restrict__ lcol,
-    const VT *__restrict__ val, int it, double tol2, T *__restrict__ x, T *__restrict__ p, const T *__restrict__ rin,
+    RbCsr<VT> M, int it, double tol2, T *__restrict__ x, T *__restrict__ p, const T *__restrict__ rin,
     T *__restrict__ rout, const T *__restrict__ sin, T *__restrict__ sout, const T *__restrict__ win,
     T *__restrict__ wout, const T *__restrict__ dinv, const double *__restrict__ gin, int ng,
     const double *__restrict__ din, int nd, double *__restrict__ gout, double *__restrict__ dout,
     double *__restrict__ sc, int *__restrict__ flag) {
-  constexpr int PER = NNZB / NT;
-  __shared__ double lds[NNZB * sizeof(T) / sizeof(double)];
-  T *xs = reinterpret_cast<T *>(lds);
-  T *prod = xs;
-  double *sh = lds;
+  __shared__ RbLds<T, NNZB, NT> lds;
+  double *sh = lds.red;
   if (*flag) return;
   double g, d;
   sum_parts2(gin, ng, din, nd, sh, g, d);
@@ -3199,75 +3234,12 @@ __global__ void __launch_bounds__(NT) k_scg_fused(
   };
   // a grid of at most SCG_MAX_GRID blocks walks all row blocks, so the partials every block sums
   // stay few however large the matrix is
-  for (int64_t rbk = lb; rbk < nrblk; rbk += gridDim.x) {
-    const int32_t r0 = rblk[rbk], r1 = rblk[rbk + 1];
-    const int32_t j0 = rp[r0], j1 = rp[r1];
-    const int nz = j1 - j0;
-    const int nrows = r1 - r0;
-    __syncthreads();  // sh (the partial sums above) and the last row block's products alias the staging buffer
-    if (nz <= NNZB) {
-      const int ri0 = threadIdx.x >> 2, q = threadIdx.x & 3;
-      int a0 = 0, e0 = 0;
-      if (ri0 < nrows) {
-        a0 = rp[r0 + ri0] - j0;
-        e0 = rp[r0 + ri0 + 1] - j0;
-      }
-      int li[PER];
-      T vv[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int t = threadIdx.x + k * NT;
-        li[k] = -1;
-        vv[k] = (T)0;
-        if (t < nz) {
-          li[k] = lcol[j0 + t];
-          vv[k] = (T)val[j0 + t];
-        }
-      }
-      const int u0 = ubase[rbk], nu = ubase[rbk + 1] - u0;
-      for (int base = 0; base < nu; base += 2 * NT) {
-        const int t0 = base + threadIdx.x, t1 = t0 + NT;
-        const int32_t c0 = ucol[u0 + min(t0, nu - 1)], c1 = ucol[u0 + min(t1, nu - 1)];
-        const T x0 = scg_next<T>(rin, win, sin, dinv, c0, a, b, first).u;
-        const T x1 = scg_next<T>(rin, win, sin, dinv, c1, a, b, first).u;
-        if (t0 < nu) xs[t0] = x0;
-        if (t1 < nu) xs[t1] = x1;
-      }
-      __syncthreads();
-      T pv[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) pv[k] = li[k] >= 0 ? vv[k] * xs[li[k]] : (T)0;
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < PER; ++k)
-        if (li[k] >= 0) prod[threadIdx.x + k * NT] = pv[k];
-      __syncthreads();
-      for (int base = 0; base < nrows; base += NT / 4) {
-        const int ri = base + ri0;
-        int ja = a0, je = e0;
-        if (base > 0 && ri < nrows) {
-          ja = rp[r0 + ri] - j0;
-          je = rp[r0 + ri + 1] - j0;
-        }
-        T sv = (T)0;  // partial row sums in the vector type, as in csr_row_block
-        if (ri < nrows)
-          for (int t = ja + q; t < je; t += 4) sv += prod[t];
-        sv += __shfl_xor(sv, 1, 4);
-        sv += __shfl_xor(sv, 2, 4);
-        if (ri < nrows && q == 0) finish(r0 + ri, (double)sv);
-      }
-    } else {
-      // a single row longer than the staging buffer
-      double sv = 0.0;
-      for (int t = threadIdx.x; t < nz; t += NT) {
-        const int32_t c = col[j0 + t];
-        sv += (double)((T)val[j0 + t] * scg_next<T>(rin, win, sin, dinv, c, a, b, first).u);
-      }
-      sv = block_sum(sv, sh);
-      if (threadIdx.x == 0) finish(r0, sv);
-    }
+  for (int64_t rbk = lb; rbk < M.nrblk; rbk += gridDim.x) {
+    __syncthreads();  // the last row block's sums have been read
+    csr_row_block<VT, T, NNZB, NT>(
+        M, rbk, lds, [&](int32_t c) { return scg_next<T>(rin, win, sin, dinv, c, a, b, first).u; }, finish);
   }
-  __syncthreads();  // sh aliases the products
+  __syncthreads();
   ag = block_sum(ag, sh);
   ad = block_sum(ad, sh);
   if (threadIdx.x == 0) {
@@ -3339,8 +3311,7 @@ static void inner_pcg(const PcgArgs<T, VT> &q, const T *v, const double *sv, dou
     const double *din = it == 0 ? sc + 6 : dq[a];
     const int ng = it == 0 ? vg : fg, nd = it == 0 ? 1 : fg;
     k_scg_fused<T, VT, SCG_NNZB, SCG_NT><<<fg, SCG_NT, 0, st>>>(
-        rb.nrblk, rb.d_rblk.p, S->d_row_ptr.p, S->d_col.p, rb.d_ubase.p, rb.d_ucol.p, rb.d_lcol.p, val, it, tol2, x,
-        p, r[a], r[b], s[a], s[b], w[a], w[b], dinv, gin, ng, din, nd, gq[b], dq[b], sc, flag);
+        rb_csr<VT>(S, rb, val), it, tol2, x, p, r[a], r[b], s[a], s[b], w[a], w[b], dinv, gin, ng, din, nd, gq[b], dq[b], sc, flag);
   }
 }
 
@@ -3634,7 +3605,6 @@ static Matrix *krylov_operator(Matrix *A, bool mixed) {
   hipStream_t st = A->ctx->stream;
   if (mixed) {
     K->d_val32.alloc(std::max<int64_t>(K->nnz, 1));
-    ensure_row_blocks32(K);
   }
   if (A->op_version != A->version) {
     k_gather_vals<<<nblk(K->nnz), NTHR, 0, st>>>(K->nnz, K->d_src.p, A->d_val.p, K->d_val.p,
@@ -3761,7 +3731,6 @@ static void solve_gmres(Matrix *A, Precond *P, const double *b, double *x, const
   if (mixed && !P) {
     // plain GMRES in FP32 needs an FP32 copy of A
     refresh_val32(A, A->ctx->stream);
-    ensure_row_blocks32(A);
   }
   const double bn = norm_masked(A, b, w);
   double rn = residual64(A, P, b, x, w.r64.p, w);
@@ -4009,7 +3978,7 @@ static void solve_minres(Matrix *A, Precond *P, const double *b, double *x, cons
 // else A. The operator leaves out only exact zeros, so the residual is A's up to summation order.
 static Matrix *residual_operator(Matrix *A) {
   Matrix *K = A->op;
-  if (A->dg || !K || A->op_pairs != A->active_pairs || K->nnz == 0 || K->rb64.nnzb == 0) return A;
+  if (A->dg || !K || A->op_pairs != A->active_pairs || K->nnz == 0 || K->rb.nnzb == 0) return A;
   const int nb = (int)A->space->blocks.size();
   const uint64_t all = nb * nb == 64 ? ~0ull : (1ull << (nb * nb)) - 1;
   if (A->active_pairs == 0 || (A->active_pairs & all) == all) return A;
@@ -4080,18 +4049,19 @@ void residual_norms_noalloc(Matrix *A0, const double *b, const double *x, double
   Ctx *ctx = A->ctx;
   double *sp = ctx->noalloc_scratch;
   OCMP_REQUIRE(sp != nullptr, "the context has no allocation-free scratch");
-  OCMP_REQUIRE(A->rb64.nnzb != 0, "the matrix has no SpMV row blocks");
+  OCMP_REQUIRE(A->rb.nnzb != 0, "the matrix has no SpMV row blocks");
   hipStream_t st = ctx->stream;
   const int grid = spmv_grid(A);
   const int dgrid = red_grid(A->n);
   // [0, grid): SpMV partials; [grid, grid + SEG_BLOCKS): second-stage sums of a long reduction;
   // then dgrid partials of ||b||^2
-  const int64_t need = (int64_t)grid + SEG_BLOCKS + dgrid;
+  // (counted as one partial per SPMV_NNZB nonzeros, so the limit does not depend on the block size)
+  const int64_t need = std::max<int64_t>(grid, A->nnz / SPMV_NNZB) + SEG_BLOCKS + dgrid;
   if (need > NOALLOC_SCRATCH_DOUBLES)
     throw Error(OCMP_ERR_ARG, "residual_norms_noalloc: the matrix needs " + std::to_string(need) +
                                   " doubles of scratch, more than the " + std::to_string(NOALLOC_SCRATCH_DOUBLES) +
                                   " of the static array (at most about " +
-                                  std::to_string((NOALLOC_SCRATCH_DOUBLES - SEG_BLOCKS - MAX_RED_BLOCKS) * SPMV_NNZB64) +
+                                  std::to_string((NOALLOC_SCRATCH_DOUBLES - SEG_BLOCKS - MAX_RED_BLOCKS) * SPMV_NNZB) +
                                   " nonzeros)");
   spmv_dispatch<double, double>(A, A->d_val.p, x, (double *)nullptr, b, A->space->d_free.p, (const double *)nullptr,
                                 nullptr, 1, sp, grid, st);

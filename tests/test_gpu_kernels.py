@@ -80,6 +80,85 @@ def test_load_vector_blocks_and_facets(gpu_ctx):
     assert float(none.vec.abs().max()) == 0.0
 
 
+# ------------------------------------------------------------------------------------------ SpMV row blocks
+
+
+def fan(n):
+    """n triangles around one vertex: its P3 row has 6 n + 1 nonzeros per component (at most 256 triangles,
+    the space's colours)."""
+    from opencmp_amd.mesh import Mesh
+    t = 2 * np.pi * np.arange(n) / n
+    ring = np.stack([np.cos(t), np.sin(t)], 1)
+    k = np.arange(n)
+    el = np.stack([np.zeros(n, int), 1 + k, 1 + (k + 1) % n], 1).astype(np.int32)
+    return Mesh(np.concatenate([[[0.0, 0.0]], ring]), el, el[:, 1:].copy(), np.zeros(n, np.int32), ['rim'])
+
+
+def shuffled(m, seed):
+    """The mesh with its vertices renumbered at random: neighbouring rows share few columns."""
+    from opencmp_amd.mesh import Mesh
+    p = np.random.default_rng(seed).permutation(m.nv)
+    c = np.empty_like(m.coords)
+    c[p] = m.coords
+    return Mesh(c, p[m.elems].astype(np.int32), p[m.bnd_facets].astype(np.int32), m.bnd_markers, m.bnd_names)
+
+
+@pytest.mark.parametrize('name,make,order', [
+    ('one block', lambda: unit_square(1), 1),
+    ('several small blocks', lambda: unit_square(23), 3),
+    ('large blocks', lambda: unit_cube(15), 3),
+    ('rows of 4,503 nonzeros', lambda: fan(250), (3, 3)),
+    ('rows of 2,042 nonzeros, longer than a block', lambda: fan(170), (3, 2)),
+    ('rows of 2,030 nonzeros, each a block', lambda: fan(169), (3, 2)),
+    ('blocks with too many distinct columns', lambda: shuffled(unit_square(310), 1), 2),
+])
+def test_spmv_row_blocks(gpu_ctx, name, make, order):
+    """y = A x against scipy on the same values: rows of at most 4,503 terms, 1e-14 relative."""
+    import torch
+    C = core()
+    order, ncomp = order if isinstance(order, tuple) else (order, 1)
+    fes = C.FESpace(C.Mesh(make(), gpu_ctx), [C.H1(order)] * ncomp)
+    a = C.BilinearForm(fes, [C.Vol(k, i, i, coef=c) for i in range(ncomp) for k, c in (('gradgrad', 1.0), ('mass', 3.0))])
+    a.Assemble()
+    x = np.random.default_rng(2).standard_normal(fes.ndof)
+    y = gpu_ctx.zeros(fes.ndof)
+    a.mult(torch.tensor(x, device='cuda'), y)
+    ref = a.to_scipy() @ x
+    assert rel(y.cpu().numpy(), ref) < 1e-14
+    if fes.ndof > 1000:
+        # FP32 blocks inside FP64 refinement
+        f = C.LinearForm(fes, [C.Source(0, (L.FN_CONST, (1.0,)))])
+        f.Assemble()
+        pre = C.Preconditioner(a, 'local', precision='mixed')
+        pre.Update()
+        u = C.GridFunction(fes)
+        r = C.solve(a, f.vec, u.vec, pre, 'CG', tol=1e-10, precision='mixed')
+        assert r.converged and r.rel_residual <= 1e-10
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+def test_spmv_rows_without_nonzeros(gpu_ctx, precision):
+    """FGMRES multiplies by the operator without untouched block pairs: with terms on one of two
+    components, half of its rows are empty. The solution equals that of the one component alone."""
+    C = core()
+    hm = unit_square(9)
+    sol = []
+    for comps in ([C.H1(2, 'left'), C.H1(2, 'left')], [C.H1(2, 'left')]):
+        fes = C.FESpace(C.Mesh(hm, gpu_ctx), comps)
+        a = C.BilinearForm(fes, [C.Vol('gradgrad', 0, 0), C.Vol('mass', 0, 0)])
+        f = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, POLY[2]))])
+        a.Assemble()
+        f.Assemble()
+        pre = C.Preconditioner(a, 'local', precision=precision)
+        pre.Update()
+        u = C.GridFunction(fes)
+        r = C.solve(a, f.vec, u.vec, pre, 'FGMRes', tol=1e-12, precision=precision, restart=60, inner_tol=1e-4)
+        assert r.converged
+        sol.append(u.vec.cpu().numpy())
+    n = len(sol[1])
+    assert rel(sol[0][:n], sol[1]) < 1e-10 and not sol[0][n:].any()
+
+
 # ------------------------------------------------------------------------------------------ U-net
 
 
