@@ -1331,80 +1331,100 @@ void build_h1_gather(Matrix *A) {
         fill[r]++;
       }
   }
-  int maxrow = 0, maxent = 0;
-  for (int64_t r = 0; r < n; ++r) {
-    maxrow = std::max(maxrow, A->row_ptr[r + 1] - A->row_ptr[r]);
-    maxent = std::max(maxent, pptr[r + 1] - pptr[r]);
-  }
-  OCMP_REQUIRE(maxrow <= 65536, "a row with more than 65536 nonzeros");
-  const bool narrow = maxrow <= 256;
-  const int sb = narrow ? 1 : 2;
-  // row blocks: staged values (entries x nl doubles + positions) of about 28 KB and at most 2048
-  // nonzeros per block, greedily over consecutive rows; a row that alone exceeds that gets a block
-  // of its own and the buffers grow to it, up to 48 KB of LDS in all
-  const int emax = std::max(std::max(1, 12288 / (nl * (8 + sb) + 2)), maxent);
-  const int accmax = std::max(1024, maxrow);
-  A->gblk.clear();
-  A->maxrow = maxrow;
+  int maxent = 0;
+  for (int64_t r = 0; r < n; ++r) maxent = std::max(maxent, pptr[r + 1] - pptr[r]);
+  // row blocks: staged values and their list (10 bytes each) of about 24 KB, greedily over
+  // consecutive rows (12, 16, 24 and 40 KB: 767, 626, 565 and 709 us on 62M 3D P3 nonzeros, 597, 605,
+  // 600 and 748 on 53M of the INS channel, 570, 414, 400 and 528 on 20M of 3D diffuse-interface
+  // Stokes); a row that alone exceeds that gets a block of its own and the buffers grow to it, up to
+  // 48 KB of LDS in all
+  const int emax = std::max(std::max(1, 24576 / (nl * 10)), maxent);
   A->gemax = emax;
-  A->gaccmax = accmax;
   A->npatch = np;
-  if ((size_t)emax * (nl * (8 + sb) + 2) + (size_t)accmax * 8 > 49152 || emax > 65535) return;  // colour path
-  A->gblk.push_back(0);
+  A->ngblk = 0;
+  if ((size_t)emax * (nl * 10 + 4) > 49152) return;  // colour path
+  std::vector<int32_t> gblk(1, 0);
   for (int64_t r = 0; r < n;) {
     int64_t r1 = r + 1;
-    while (r1 < n && pptr[r1 + 1] - pptr[r] <= emax && A->row_ptr[r1 + 1] - A->row_ptr[r] <= accmax) ++r1;
-    A->gblk.push_back((int32_t)r1);
+    while (r1 < n && pptr[r1 + 1] - pptr[r] <= emax) ++r1;
+    gblk.push_back((int32_t)r1);
     r = r1;
   }
-  const int64_t nblk = (int64_t)A->gblk.size() - 1;
-  // per block: entries sorted by local row (stable), their positions, and each entry's column
-  // positions within its row
+  const int64_t nblk = (int64_t)gblk.size() - 1;
+  // per block: entries sorted by local row (stable), and for every nonzero the staged values it sums,
+  // in the rows' element order
   std::vector<int32_t> spe(np);
-  std::vector<uint8_t> spli(np);
-  std::vector<uint16_t> gpos(np), gloff((size_t)nblk * (nl + 1));
-  std::vector<uint8_t> s8(narrow ? (size_t)np * nl : 0);
-  std::vector<uint16_t> s16(narrow ? 0 : (size_t)np * nl);
-#pragma omp parallel for schedule(dynamic, 64)
+  std::vector<GatherBlk> desc(nblk);
+  int64_t ix8 = 0;
   for (int64_t b = 0; b < nblk; ++b) {
-    const int32_t r0 = A->gblk[b], r1 = A->gblk[b + 1];
-    const int32_t e0 = pptr[r0], ne = pptr[r1] - e0;
-    std::vector<int> cnt(nl + 1, 0);
-    for (int32_t k = 0; k < ne; ++k) cnt[pli[e0 + k] + 1]++;
-    for (int L = 0; L < nl; ++L) cnt[L + 1] += cnt[L];
-    for (int L = 0; L <= nl; ++L) gloff[(size_t)b * (nl + 1) + L] = (uint16_t)cnt[L];
-    std::vector<int> fill(cnt.begin(), cnt.end() - 1);
-    for (int32_t r = r0; r < r1; ++r) {
-      const int32_t *c0 = A->col.data() + A->row_ptr[r];
-      const int32_t *c1 = A->col.data() + A->row_ptr[r + 1];
-      for (int32_t p = pptr[r]; p < pptr[r + 1]; ++p) {
-        const int q = fill[pli[p]]++;             // sorted position within the block
-        gpos[p] = (uint16_t)q;
-        const int64_t sp = e0 + q;
-        spe[sp] = pe[p];
-        spli[sp] = pli[p];
-        const int32_t *ed = &s.edofs[(int64_t)pe[p] * nl];
-        for (int j = 0; j < nl; ++j) {
-          const int pos = (int)(std::lower_bound(c0, c1, ed[j]) - c0);
-          if (narrow)
-            s8[(size_t)sp * nl + j] = (uint8_t)pos;
-          else
-            s16[(size_t)sp * nl + j] = (uint16_t)pos;
+    const int32_t r0 = gblk[b], r1 = gblk[b + 1];
+    desc[b] = GatherBlk{pptr[r0], pptr[r1] - pptr[r0], A->row_ptr[r0], A->row_ptr[r1] - A->row_ptr[r0], 0, 0,
+                        (int32_t)ix8, 0};
+    ix8 += ((int64_t)desc[b].ne * nl + 7) / 8;
+  }
+  OCMP_REQUIRE(ix8 < INT32_MAX, "too many element entries");
+  std::vector<uint16_t> gend(A->nnz), gidx((size_t)ix8 * 8, 0);
+  std::vector<std::vector<uint32_t>> units(nblk);
+  std::vector<std::unique_ptr<int32_t, void (*)(void *)>> pos_of;  // per thread: a row's column -> its position
+  for (int t = 0; t < omp_get_max_threads(); ++t) {
+    pos_of.emplace_back((int32_t *)std::malloc(std::max<int64_t>(n, 1) * sizeof(int32_t)), std::free);
+    if (!pos_of.back()) throw std::bad_alloc();
+  }
+#pragma omp parallel
+  {
+    int32_t *const pos = pos_of[omp_get_thread_num()].get();
+    std::vector<int> cnt, fill;
+    std::vector<int32_t> zof, start;
+#pragma omp for schedule(static)
+    for (int64_t b = 0; b < nblk; ++b) {
+      const int32_t r0 = gblk[b], r1 = gblk[b + 1];
+      const int32_t e0 = desc[b].e0, ne = desc[b].ne, z0 = desc[b].z0, nz = desc[b].nz;
+      uint16_t *const ix = gidx.data() + (size_t)desc[b].ix8 * 8;
+      cnt.assign(nl + 1, 0);
+      for (int32_t k = 0; k < ne; ++k) cnt[pli[e0 + k] + 1]++;
+      for (int L = 0; L < nl; ++L) cnt[L + 1] += cnt[L];
+      for (int L = 0; L < nl; ++L)
+        for (int g = cnt[L]; g < cnt[L + 1]; g += 16)
+          units[b].push_back((uint32_t)L | (uint32_t)(std::min(16, cnt[L + 1] - g) - 1) << 6 | (uint32_t)g << 10);
+      fill.assign(cnt.begin(), cnt.end() - 1);
+      zof.resize((size_t)ne * nl);
+      start.assign(nz + 1, 0);
+      for (int32_t r = r0; r < r1; ++r) {
+        for (int32_t k = A->row_ptr[r]; k < A->row_ptr[r + 1]; ++k) pos[A->col[k]] = k - z0;
+        for (int32_t p = pptr[r]; p < pptr[r + 1]; ++p) {
+          const int32_t *ed = &s.edofs[(int64_t)pe[p] * nl];
+          for (int j = 0; j < nl; ++j) {
+            const int32_t z = pos[ed[j]];
+            zof[(size_t)(p - e0) * nl + j] = z;
+            start[z + 1]++;
+          }
         }
+      }
+      for (int32_t z = 0; z < nz; ++z) {
+        start[z + 1] += start[z];
+        gend[(size_t)z0 + z] = (uint16_t)start[z + 1];
+      }
+      for (int32_t p = 0; p < ne; ++p) {
+        const int q = fill[pli[e0 + p]]++;  // sorted position within the block
+        spe[e0 + q] = pe[e0 + p];
+        for (int j = 0; j < nl; ++j)
+          ix[start[zof[(size_t)p * nl + j]]++] = (uint16_t)(q * nl + j);
       }
     }
   }
+  std::vector<uint32_t> gunit;
+  for (int64_t b = 0; b < nblk; ++b) {
+    desc[b].u0 = (int32_t)gunit.size();
+    desc[b].nu = (int32_t)units[b].size();
+    gunit.insert(gunit.end(), units[b].begin(), units[b].end());
+  }
   hipStream_t st = A->ctx->stream;
-  A->d_pptr.upload(pptr, st);
+  A->ngblk = nblk;
+  A->d_gunit.upload(gunit, st);
+  A->d_gblk.upload(desc, st);
   A->d_pe.upload(spe, st);
-  A->d_pli.upload(spli, st);
-  A->d_gpos.upload(gpos, st);
-  A->d_gloff.upload(gloff, st);
-  A->d_gblk.upload(A->gblk, st);
-  if (narrow)
-    A->d_pslot8.upload(s8, st);
-  else
-    A->d_pslot16.upload(s16, st);
+  A->d_gend.upload(gend, st);
+  A->d_gidx.upload(gidx, st);
   OCMP_HIP(hipStreamSynchronize(st));
 }
 

@@ -250,6 +250,14 @@ struct RowBlocks {
   int64_t nrblk = 0, nucol = 0;
 };
 
+struct GatherBlk {
+  int32_t e0, ne;      // entries
+  int32_t z0, nz;      // nonzeros
+  int32_t u0, nu;      // units
+  int32_t ix8;         // first entry of d_gidx, in eights (each block's part is padded to them)
+  int32_t pad;
+};
+
 struct Work;                  // a matrix' Krylov scratch (linalg.hip), created on first solve
 void work_release(Work *w);   // frees it (device buffers, pinned host buffer, events)
 
@@ -264,25 +272,17 @@ struct Matrix {
   // H1 boundary-facet scatter: element -> CSR slot map (colours live in the space), built on the
   // first assembly with boundary terms
   DBuf<int32_t> d_slot;              // nel*nloc*nloc
-  // H1 row-owner gather (volume terms): per CSR row its element entries in element order
-  // (patch), every entry's compound local row index and the position in the row of each of the
-  // element's nloc columns (1 byte when every row has at most 256 nonzeros, else 2)
-  DBuf<int32_t> d_pptr;              // n+1
+  // H1 row-owner gather (volume terms): blocks of consecutive rows with at most gemax element
+  // entries (element, local row), sorted by local row; empty when the entries of one row do not fit in
+  // LDS. Units of a block: at most 16 entries of one local row. Nonzero t of a block sums the
+  // element-row values V[entry][column] listed in its part of d_gidx, from the previous nonzero's
+  // d_gend to its own.
+  DBuf<GatherBlk> d_gblk;
   DBuf<int32_t> d_pe;                // entries: element
-  DBuf<uint8_t> d_pslot8;            // entries x nloc (maxrow <= 256)
-  DBuf<uint16_t> d_pslot16;          // entries x nloc (maxrow > 256)
-  int64_t npatch = 0;
-  int maxrow = 0;
-  // row blocks of the gather: rows [gblk[b], gblk[b+1]) with at most gemax element entries and
-  // gaccmax nonzeros (staged in LDS); empty when some row alone would not fit. Within a block the
-  // entries are stored sorted by local row index (d_pe, d_pslot in that order): d_gloff[b*(nl+1)+L]
-  // is where local row L starts (relative to the block's first entry), d_gpos[p] the sorted position
-  // of the p-th entry in row order (pptr indexes row order)
-  std::vector<int32_t> gblk;
-  DBuf<int32_t> d_gblk;
-  DBuf<uint16_t> d_gpos, d_gloff;
-  DBuf<uint8_t> d_pli;               // sorted entries: local row index
-  int gemax = 0, gaccmax = 0;
+  DBuf<uint32_t> d_gunit;            // units: local row | (entries - 1) << 6 | first entry << 10
+  DBuf<uint16_t> d_gend, d_gidx;
+  int64_t ngblk = 0, npatch = 0;
+  int gemax = 0;
   DBuf<double> d_factors;            // nel x (factors per element) of the last assembly
   DBuf<int32_t> d_dslot;             // n: CSR slot of the diagonal entry (-1: none), built on first use
   DBuf<char> d_gdesc;                // the gather's kernel descriptors

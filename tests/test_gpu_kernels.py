@@ -159,6 +159,45 @@ def test_spmv_rows_without_nonzeros(gpu_ctx, precision):
     assert rel(sol[0][:n], sol[1]) < 1e-10 and not sol[0][n:].any()
 
 
+# ------------------------------------------------------------------------------------------ row gather
+
+
+@pytest.mark.parametrize('make,order', [
+    (lambda: unit_square(1), 1), (lambda: unit_square(6), 2), (lambda: unit_cube(2), 1), (lambda: unit_cube(3), 3),
+    (lambda: fan(16), 3),     # exactly one unit of 16 entries for the centre's row
+    (lambda: fan(17), 2),     # and one entry more
+    (lambda: fan(200), 3),    # a block grown to one row's 200 entries
+    (lambda: fan(250), 3),    # more than LDS takes: the element scatter
+])
+def test_gather_units(gpu_ctx, make, order):
+    """Matrix values against the oracle's quadrature, written, accumulated in a second launch (33 terms)
+    and with coefficients that make terms share a table or not (relative Frobenius 1e-13)."""
+    C = core()
+    hm = make()
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.H1(order), C.H1(1)])
+    t = fem.Topology(hm)
+    cs = fem.Compound([fem.Space(t, 'H1', order), fem.Space(t, 'H1', 1)])
+
+    def ref(g, m, c):
+        A = fem.Assembler(cs)
+        fem.assemble_volume(A, [dict(kind='grad_grad', trial=0, test=0, coef=g),
+                                dict(kind='mass', trial=0, test=0, coef=m),
+                                dict(kind='mass', trial=1, test=0, coef=c)])
+        return A.matrix().data
+
+    def gpu(terms):
+        a = C.BilinearForm(fes, terms)
+        a.Assemble()
+        return a.values()
+
+    G, M, X = (lambda c: C.Vol('gradgrad', 0, 0, coef=c)), (lambda c: C.Vol('mass', 0, 0, coef=c)), \
+        (lambda c: C.Vol('mass', 1, 0, coef=c))
+    assert rel(gpu([G(2.0), M(3.0), X(0.5)]), ref(2.0, 3.0, 0.5)) < 1e-13
+    assert rel(gpu([G(2.0), G(2.0), M(0.5), X(0.5)]), ref(4.0, 0.5, 0.5)) < 1e-13
+    assert rel(gpu([G(2.0), G(1.0), M(0.5), X(0.25)]), ref(3.0, 0.5, 0.25)) < 1e-13
+    assert rel(gpu([G(1.0)] * 31 + [M(1.0), X(1.0)]), ref(31.0, 1.0, 1.0)) < 1e-13
+
+
 # ------------------------------------------------------------------------------------------ U-net
 
 
