@@ -916,22 +916,70 @@ __global__ void __launch_bounds__(NTHR) k_dot(int64_t n, const T *__restrict__ a
   if (threadIdx.x == 0) part[lb] = s;
 }
 
-// CG update with device scalars: alpha = rz[it&1] / pq
-// x += alpha p; r -= alpha q; z = dinv r; partials of r.z and r.r
+// sums of two partial arrays, the same in every block (and every thread)
+__device__ __forceinline__ void sum_parts2(const double *__restrict__ pa, int na, const double *__restrict__ pb,
+                                           int nb, double *sh, double &sa, double &sb) {
+  double a[8], b[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    const double va = pa[min(i, na - 1)], vb = pb[min(i, nb - 1)];
+    a[k] = i < na ? va : 0.0;
+    b[k] = i < nb ? vb : 0.0;
+  }
+  for (int i = threadIdx.x + 8 * blockDim.x; i < na; i += blockDim.x) a[0] += pa[i];
+  for (int i = threadIdx.x + 8 * blockDim.x; i < nb; i += blockDim.x) b[0] += pb[i];
+  double x = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  double y = ((b[0] + b[1]) + (b[2] + b[3])) + ((b[4] + b[5]) + (b[6] + b[7]));
+  x = wave_sum(x);
+  y = wave_sum(y);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  if (lane == 0) {
+    sh[wid] = x;
+    sh[nw + wid] = y;
+  }
+  __syncthreads();
+  x = 0.0;
+  y = 0.0;
+  for (int w = 0; w < nw; ++w) {
+    x += sh[w];
+    y += sh[nw + w];
+  }
+  __syncthreads();
+  sa = x;
+  sb = y;
+}
+
+// The CG recurrences between two products with A, as two launches whose blocks sum the partial sums
+// of the launch before themselves instead of waiting for reductions in between (one launch each
+// and a gap each: six launches an iteration before, three or four now, two in the small form below).
+// Scalars sc: [0], [1] r.z of even and odd iterations, [2] p.q.
+//
+// alpha = r.z / p.q; r -= alpha q; z = dinv r; partials of r.z and r.r. npq > 0: p.q is the sum of
+// that many partials in pqpart (block 0 stores it for the next launch), else sc[2]. x (may be NULL)
+// += alpha p.
 template <typename T>
-__global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x, T *__restrict__ r,
-                                                    T *__restrict__ z, const T *__restrict__ p,
-                                                    const T *__restrict__ q, const T *__restrict__ dinv,
-                                                    const double *__restrict__ sc, int it, double *__restrict__ part) {
-  __shared__ double sh[NTHR / 64];
-  const double alpha_d = sc[it & 1] / sc[2];
-  const T alpha = (T)alpha_d;
+__global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x, const T *__restrict__ p,
+                                                    T *__restrict__ r, T *__restrict__ z, const T *__restrict__ q,
+                                                    const T *__restrict__ dinv, double *__restrict__ sc, int it,
+                                                    const double *__restrict__ pqpart, int npq,
+                                                    double *__restrict__ part) {
+  __shared__ double sh[2 * NTHR / 64];
+  double pq;
+  if (npq > 0) {
+    double none;
+    sum_parts2(pqpart, npq, pqpart, 1, sh, pq, none);
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[2] = pq;
+  } else {
+    pq = sc[2];
+  }
+  const T alpha = (T)(sc[it & 1] / pq);
   const int lb = xcd_block();
   const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
   const int64_t i0 = lb * chunk, i1 = min(n, i0 + chunk);
   double rz = 0.0, rr = 0.0;
   for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    x[i] += alpha * p[i];
+    if (x) x[i] += alpha * p[i];
     const T ri = r[i] - alpha * q[i];
     r[i] = ri;
     const T zi = dinv[i] * ri;
@@ -947,13 +995,80 @@ __global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x
   }
 }
 
-// p = z + beta p, beta = rz[(it+1)&1] / rz[it&1]
+// x += alpha p; p = z + beta p, beta = (new r.z) / r.z; block 0 stores the new r.z and r.r (hist)
 template <typename T>
-__global__ void k_cg_p(int64_t n, T *__restrict__ p, const T *__restrict__ z, const double *__restrict__ sc, int it) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T beta = (T)(sc[(it + 1) & 1] / sc[it & 1]);
-  p[i] = z[i] + beta * p[i];
+__global__ void __launch_bounds__(NTHR) k_cg_p(int64_t n, T *__restrict__ x, T *__restrict__ p, const T *__restrict__ z,
+                                               double *__restrict__ sc, int it, const double *__restrict__ part,
+                                               int np, double *__restrict__ hist) {
+  __shared__ double sh[2 * NTHR / 64];
+  const double old = sc[it & 1];
+  const T alpha = (T)(old / sc[2]);
+  double rz, rr;
+  sum_parts2(part, np, part + np, np, sh, rz, rr);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[(it + 1) & 1] = rz;
+    hist[0] = rr;
+  }
+  const T beta = (T)(rz / old);
+  const int lb = xcd_block();
+  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
+  const int64_t i0 = lb * chunk, i1 = min(n, i0 + chunk);
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
+    const T pi = p[i];
+    x[i] += alpha * pi;
+    p[i] = z[i] + beta * pi;
+  }
+}
+
+// The small form: p = z + beta p_old is formed inside the product, where a block needs it (its rows,
+// and its columns: pointwise, by the same expression as the owner), so an iteration is this launch and
+// k_cg_update. beta comes from that launch's np partials of r.z and r.r; it = 0: p = z. hist: where
+// block 0 stores the r.r of the iteration before (NULL at the first).
+template <typename VT, typename T>
+__global__ void __launch_bounds__(NTHR) k_cg_spmv(RbCsr<VT> M, const T *__restrict__ z, const T *__restrict__ pin,
+                                                  T *__restrict__ pout, T *__restrict__ q,
+                                                  const uint8_t *__restrict__ mask, double *__restrict__ sc, int it,
+                                                  const double *__restrict__ part, int np, double *__restrict__ hist,
+                                                  double *__restrict__ pqpart) {
+  __shared__ RbLds<T, SPMV_NNZB, NTHR> lds;
+  const bool first = it == 0;
+  T beta = (T)0;
+  if (!first) {
+    double rz, rr;
+    sum_parts2(part, np, part + np, np, lds.red, rz, rr);
+    beta = (T)(rz / sc[(it + 1) & 1]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc[it & 1] = rz;
+      if (hist) hist[0] = rr;
+    }
+  }
+  const int lb = xcd_block();
+  double acc = 0.0;
+  auto pnew = [&](int64_t c) { return first ? z[c] : z[c] + beta * pin[c]; };
+  if (lb < M.nrblk)
+    csr_row_block<VT, T, SPMV_NNZB, NTHR>(
+        M, lb, lds, [&](int32_t c) { return pnew(c); },
+        [&](int64_t r, double s) {
+          const T pr = pnew(r), v = mask[r] ? (T)s : (T)0;
+          pout[r] = pr;
+          q[r] = v;
+          acc += (double)pr * (double)v;
+        });
+  __syncthreads();
+  acc = block_sum(acc, lds.red);
+  if (threadIdx.x == 0) pqpart[lb] = acc;
+}
+
+// the r.z and r.r of a batch's last iteration
+__global__ void __launch_bounds__(NTHR) k_cg_tail(double *__restrict__ sc, int it, const double *__restrict__ part, int np,
+                                                  double *__restrict__ hist) {
+  __shared__ double sh[2 * NTHR / 64];
+  double rz, rr;
+  sum_parts2(part, np, part + np, np, sh, rz, rr);
+  if (threadIdx.x == 0) {
+    sc[it & 1] = rz;
+    hist[0] = rr;
+  }
 }
 
 // z = dinv * r (with optional scale), p = z
@@ -1337,7 +1452,24 @@ static void ensure_part(Work &w, size_t n) {
   w.part.alloc(std::max<size_t>(w.part.n, std::max<size_t>(n, (size_t)68 * MAX_RED_BLOCKS)));
 }
 
-// first stage of a long reduction: block s sums part[s*seg, (s+1)*seg) into out[s]
+// one long row of partial sums by one large block, several loads of a thread in flight (10,600 partials:
+// 4.6 us; two launches of 1024 and one blocks before: 9.4 us)
+__global__ void __launch_bounds__(1024) k_reduce_long(const double *__restrict__ part, int64_t nparts,
+                                                      double *__restrict__ out, int do_sqrt) {
+  __shared__ double sh[1024 / 64];
+  double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int64_t b = threadIdx.x; b < nparts; b += 8 * 1024) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = part[min(b + k * 1024, nparts - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] += b + k * 1024 < nparts ? v[k] : 0.0;
+  }
+  const double s = block_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])), sh);
+  if (threadIdx.x == 0) out[0] = do_sqrt ? sqrt(s) : s;
+}
+
+// first stage of a very long reduction: block s sums part[s*seg, (s+1)*seg) into out[s]
 __global__ void k_reduce_seg(const double *__restrict__ part, int64_t nparts, int64_t seg, double *__restrict__ out) {
   __shared__ double sh[NTHR / 64];
   const int64_t b0 = (int64_t)blockIdx.x * seg, b1 = min(nparts, b0 + seg);
@@ -1349,11 +1481,15 @@ __global__ void k_reduce_seg(const double *__restrict__ part, int64_t nparts, in
 
 constexpr int SEG_BLOCKS = 1024;
 
-// reduce nvals partial rows of `grid` entries into dst (device), fixed order. A single long row
+// reduce nvals partial rows of `grid` entries into dst (device), fixed order. A very long row
 // (one partial per SpMV block) is reduced in two stages through part[grid, grid + SEG_BLOCKS).
 static void reduce_to(double *part, int64_t grid, int nvals, double *dst, hipStream_t st, bool do_sqrt = false) {
-  if (grid <= 8192 || nvals != 1) {
+  if (nvals != 1 || grid <= 1024) {
     k_reduce<<<nvals, NTHR, 0, st>>>(part, (int)grid, dst, do_sqrt ? 1 : 0);
+    return;
+  }
+  if (grid <= 65536) {
+    k_reduce_long<<<1, 1024, 0, st>>>(part, grid, dst, do_sqrt ? 1 : 0);
     return;
   }
   const int64_t seg = (grid + SEG_BLOCKS - 1) / SEG_BLOCKS;
@@ -2138,16 +2274,24 @@ void precond_update_jacobi(Precond *P) {
 
 // Batches of `check` iterations are enqueued ahead; the host checks the
 // residual history of batch b while batch b+1 runs, so the GPU never idles.
+//
+// Up to CG_SMALL_BLOCKS row blocks the small form (two launches an iteration; a launch there takes
+// its latency, and its blocks sum each other's few partials); above it the product gathers p alone, and
+// up to CG_SUM_BLOCKS partials of p.q the update sums them itself. 4,225 rows FP64: 24 -> 13.4 us an
+// iteration; 912k rows of 3D P3 in FP32: 94 -> 84 us.
+constexpr int CG_SMALL_BLOCKS = 512, CG_SUM_BLOCKS = 2048;
 template <typename VT, typename T>
-static int cg_inner(Matrix *A, const VT *val, const T *dinv, T *x, T *r, T *z, T *p, T *q, double tol_rr,
+static int cg_inner(Matrix *A, const VT *val, const T *dinv, T *x, T *r, T *z, T *p, T *q, T *p2, double tol_rr,
                     int maxit, int check_every, Work &w, int &iters_done, double *last_rr) {
-  // x, r, z, p set by the caller: r = residual, z = dinv r, p = z, sc[0] = r.z
+  // x, r, z, p set by the caller: r = residual, z = dinv r, p = z, sc[0] = r.z; p2: scratch
   Ctx *ctx = A->ctx;
   hipStream_t st = ctx->stream;
   const int64_t n = A->n;
   const int sgrid = spmv_grid<VT, T>(A);
-  ensure_part(w, (size_t)sgrid + SEG_BLOCKS + 64);
-  const int vgrid = red_grid(n);
+  const bool small = sgrid <= CG_SMALL_BLOCKS;
+  const int vgrid = std::min(red_grid(n), small ? 256 : 1024);
+  ensure_part(w, (size_t)sgrid + SEG_BLOCKS + 64 + 2 * vgrid);
+  double *pqpart = w.part.p, *vpart = w.part.p + sgrid + SEG_BLOCKS + 64;
   double *sc = ctx->scal.p;  // [0],[1]: rz ring, [2]: pq
   const int H = std::max(check_every, 1);
   w.small.alloc(std::max<size_t>(w.small.n, (size_t)2 * H + 64));
@@ -2160,25 +2304,36 @@ static int cg_inner(Matrix *A, const VT *val, const T *dinv, T *x, T *r, T *z, T
   };
   std::deque<Batch> inflight;
   int it = 0, bidx = 0;
+  T *pb[2] = {p, p2};
+  const RbCsr<VT> M = rb_csr<VT>(A, A->rb, val);
   auto enqueue = [&]() {
     const int nb = std::min(H, maxit - it);
     const int half = bidx & 1;
+    double *hs = hist + half * H;
     for (int s = 0; s < nb; ++s, ++it) {
+      if (small) {
+        {
+          KTimer tm(ctx, c_spmv, csr_bytes(A, sizeof(VT), sizeof(T)));
+          k_cg_spmv<VT, T><<<sgrid, NTHR, 0, st>>>(M, z, pb[(it + 1) & 1], pb[it & 1], q, A->space->d_free.p, sc, it,
+                                                   vpart, vgrid, s ? hs + s - 1 : nullptr, pqpart);
+        }
+        KTimer tm(ctx, c_upd, 8.0 * n * sizeof(T));
+        k_cg_update<T><<<vgrid, NTHR, 0, st>>>(n, x, pb[it & 1], r, z, q, dinv, sc, it, pqpart, sgrid, vpart);
+        continue;
+      }
       {
         KTimer tm(ctx, c_spmv, csr_bytes(A, sizeof(VT), sizeof(T)));
-        spmv_dispatch<VT, T>(A, val, p, q, nullptr, A->space->d_free.p, (const T *)nullptr, nullptr, 2, w.part.p,
+        spmv_dispatch<VT, T>(A, val, p, q, nullptr, A->space->d_free.p, (const T *)nullptr, nullptr, 2, pqpart,
                              sgrid, st);
       }
-      reduce_to(w.part.p, sgrid, 1, sc + 2, st);
-      {
-        KTimer tm(ctx, c_upd, 8.0 * n * sizeof(T));
-        k_cg_update<T><<<vgrid, NTHR, 0, st>>>(n, x, r, z, p, q, dinv, sc, it, w.part.p);
-      }
-      reduce_to(w.part.p, vgrid, 1, sc + ((it + 1) & 1), st);
-      reduce_to(w.part.p + vgrid, vgrid, 1, hist + half * H + s, st);
-      k_cg_p<T><<<nblk(n), NTHR, 0, st>>>(n, p, z, sc, it);
+      if (sgrid > CG_SUM_BLOCKS) reduce_to(pqpart, sgrid, 1, sc + 2, st);
+      KTimer tm(ctx, c_upd, 10.0 * n * sizeof(T));
+      k_cg_update<T><<<vgrid, NTHR, 0, st>>>(n, (T *)nullptr, p, r, z, q, dinv, sc, it, pqpart,
+                                             sgrid > CG_SUM_BLOCKS ? 0 : sgrid, vpart);
+      k_cg_p<T><<<vgrid, NTHR, 0, st>>>(n, x, p, z, sc, it, vpart, vgrid, hs + s);
     }
-    OCMP_HIP(hipMemcpyAsync(hh + half * H, hist + half * H, nb * sizeof(double), hipMemcpyDeviceToHost, st));
+    if (small) k_cg_tail<<<1, NTHR, 0, st>>>(sc, it, vpart, vgrid, hs + nb - 1);
+    OCMP_HIP(hipMemcpyAsync(hh + half * H, hs, nb * sizeof(double), hipMemcpyDeviceToHost, st));
     OCMP_HIP(hipEventRecord(work_event(w, half), st));
     inflight.push_back({it - nb, nb, half});
     ++bidx;
@@ -2230,7 +2385,7 @@ static void solve_cg(Matrix *A, Precond *P, const double *b, double *x, const oc
   const int vgrid = red_grid(n);
   if (!mixed) {
     w.vd.alloc((size_t)4 * n);
-    double *z = w.vd.p, *p = z + n, *q = p + n;
+    double *z = w.vd.p, *p = z + n, *q = p + n, *p2 = q + n;
     double *r = w.r64.p;
     int outer = 0;
     while (true) {
@@ -2241,7 +2396,7 @@ static void solve_cg(Matrix *A, Precond *P, const double *b, double *x, const oc
       reduce_to(w.part.p, vgrid, 1, ctx->scal.p + 0, st);
       int done = 0;
       double last = 0.0;
-      cg_inner<double, double>(A, A->d_val.p, P->dinv.p, x, r, z, p, q, o.tol * o.tol * bref * bref,
+      cg_inner<double, double>(A, A->d_val.p, P->dinv.p, x, r, z, p, q, p2, o.tol * o.tol * bref * bref,
                                o.maxit - total, check, w, done, &last);
       total += done;
       rn = residual64(A, P, b, x, w.r64.p, w);  // true residual (also restarts r)
@@ -2252,8 +2407,8 @@ static void solve_cg(Matrix *A, Precond *P, const double *b, double *x, const oc
   } else {
     OCMP_REQUIRE(P->dinv32.p && A->d_val32.p, "mixed precision needs a preconditioner built with OCMP_MIXED");
     if (A->val32_version != A->version) refresh_val32(A, st);  // an update that left the copy to FGMRES
-    w.vf.alloc((size_t)5 * n);
-    float *d = w.vf.p, *r = d + n, *z = r + n, *p = z + n, *q = p + n;
+    w.vf.alloc((size_t)6 * n);
+    float *d = w.vf.p, *r = d + n, *z = r + n, *p = z + n, *q = p + n, *p2 = q + n;
     // each inner FP32 CG reduces its residual by this factor (H1 P3, 7.2M dofs: 1e-5 took 560
     // iterations in 2 refinement steps, 1e-4 570 in 3, 1e-6 610, 1e-7 670)
     const double inner = o.inner_tol > 0 ? o.inner_tol : 1e-5;
@@ -2270,7 +2425,7 @@ static void solve_cg(Matrix *A, Precond *P, const double *b, double *x, const oc
       const double need = std::max(inner, 0.5 * o.tol * bref / rn);
       int done = 0;
       double last = 0.0;
-      cg_inner<float, float>(A, A->d_val32.p, P->dinv32.p, d, r, z, p, q, need * need, o.maxit - total, check, w,
+      cg_inner<float, float>(A, A->d_val32.p, P->dinv32.p, d, r, z, p, q, p2, need * need, o.maxit - total, check, w,
                              done, &last);
       total += done;
       k_axpy64<float><<<nblk(n), NTHR, 0, st>>>(n, rn, d, x);
@@ -3121,40 +3276,6 @@ __global__ void __launch_bounds__(NTHR) k_scg_init(int64_t n, const T *__restric
     gpart[lb] = acc;
     if (blockIdx.x == 0) flag[0] = 0;
   }
-}
-
-// the two sums of sum_parts in one pass: both sets of loads in flight together, one shared round
-__device__ __forceinline__ void sum_parts2(const double *__restrict__ pa, int na, const double *__restrict__ pb,
-                                           int nb, double *sh, double &sa, double &sb) {
-  double a[8], b[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int i = threadIdx.x + k * blockDim.x;
-    const double va = pa[min(i, na - 1)], vb = pb[min(i, nb - 1)];
-    a[k] = i < na ? va : 0.0;
-    b[k] = i < nb ? vb : 0.0;
-  }
-  for (int i = threadIdx.x + 8 * blockDim.x; i < na; i += blockDim.x) a[0] += pa[i];
-  for (int i = threadIdx.x + 8 * blockDim.x; i < nb; i += blockDim.x) b[0] += pb[i];
-  double x = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-  double y = ((b[0] + b[1]) + (b[2] + b[3])) + ((b[4] + b[5]) + (b[6] + b[7]));
-  x = wave_sum(x);
-  y = wave_sum(y);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if (lane == 0) {
-    sh[wid] = x;
-    sh[nw + wid] = y;
-  }
-  __syncthreads();
-  x = 0.0;
-  y = 0.0;
-  for (int w = 0; w < nw; ++w) {
-    x += sh[w];
-    y += sh[nw + w];
-  }
-  __syncthreads();
-  sa = x;
-  sb = y;
 }
 
 // One Chronopoulos-Gear iteration in one launch (row blocks of SCG_NNZB = 4096 nonzeros, 512 threads:
