@@ -51,6 +51,52 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
+// Sums of N values over the wave, several at a time: at each exchange a lane passes on one half of its
+// values and keeps the sums of the other, so N values take about 2 N exchanges instead of 6 N (from
+// an odd count on, plain exchanges). Afterwards lane l holds N >> h sums in v[0..), those of the values
+// from `first` on, h = the halvings; its lower 6 - h bits do not matter.
+constexpr int wave_halvings(int n) { return n > 1 && n % 2 == 0 ? 1 + wave_halvings(n / 2) : 0; }
+template <int NV, int N = NV, int O = 32>
+__device__ __forceinline__ void wave_sums(double (&v)[NV], int lane, int &first) {
+  if constexpr (O > 0) {
+    if constexpr (N > 1 && N % 2 == 0) {
+      const bool up = lane & O;
+#pragma unroll
+      for (int i = 0; i < N / 2; ++i) {
+        const double pass = up ? v[i] : v[i + N / 2], keep = up ? v[i + N / 2] : v[i];
+        v[i] = keep + __shfl_xor(pass, O, 64);
+      }
+      first += up ? N / 2 : 0;
+      wave_sums<NV, N / 2, O / 2>(v, lane, first);
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] += __shfl_xor(v[i], O, 64);
+      wave_sums<NV, N, O / 2>(v, lane, first);
+    }
+  }
+}
+
+// the block's sums of every thread's NV values: part[i * stride] for i < live, i = 0..NV-1 (NV at most the
+// block's size); sh holds NV values per wave
+template <int NV>
+__device__ __forceinline__ void block_sums(double (&v)[NV], double (*sh)[NV], int live, double *__restrict__ part,
+                                           int64_t stride) {
+  constexpr int H = wave_halvings(NV) < 6 ? wave_halvings(NV) : 6;
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  int first = 0;
+  wave_sums<NV>(v, lane, first);
+  if ((lane & ((1 << (6 - H)) - 1)) == 0) {
+#pragma unroll
+    for (int i = 0; i < (NV >> H); ++i) sh[threadIdx.x >> 6][first + i] = v[i];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < live) {
+    double s = 0.0;
+    for (int w = 0; w < nw; ++w) s += sh[w][threadIdx.x];
+    part[threadIdx.x * stride] = s;
+  }
+}
+
 // sum over the block; valid in thread 0
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   v = wave_sum(v);
@@ -1150,18 +1196,7 @@ __global__ void __launch_bounds__(NTHR) k_mdot(int64_t n, const T *__restrict__ 
       for (int c = 0; c < KE; ++c) acc[c] += (double)rows[c][i] * wi;
     }
   }
-#pragma unroll
-  for (int c = 0; c < KE; ++c) {
-    const double v = wave_sum(acc[c]);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][c] = v;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < kend) {
-    double s = 0.0;
-#pragma unroll
-    for (int wv = 0; wv < NTHR / 64; ++wv) s += sh[wv][threadIdx.x];
-    part[(int64_t)(k0 + threadIdx.x) * gridDim.x + lb] = s;
-  }
+  block_sums<KE>(acc, sh, kend, part + (int64_t)k0 * gridDim.x + lb, gridDim.x);
 }
 
 // the grid of k_mdot<T, KE>: at most the blocks that are resident together (the kernel's occupancy,
@@ -2685,20 +2720,12 @@ __global__ void __launch_bounds__(NTHR) k_bdot(int64_t n, const T *__restrict__ 
 #pragma unroll
         for (int t = 0; t < CA_S; ++t)
           acc[c][t] += (Acc)Q[(int64_t)min(q0 + c, nq - 1) * ldv + i] * (Acc)W[(int64_t)t * ldv + i];
+  double v[CA_KQ * CA_S];
 #pragma unroll
   for (int c = 0; c < CA_KQ; ++c)
 #pragma unroll
-    for (int t = 0; t < CA_S; ++t) {
-      const double v = wave_sum((double)acc[c][t]);
-      if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][c * CA_S + t] = v;
-    }
-  __syncthreads();
-  if ((int)threadIdx.x < nqt * CA_S) {
-    double sum = 0.0;
-#pragma unroll
-    for (int wv = 0; wv < NTHR / 64; ++wv) sum += sh[wv][threadIdx.x];
-    part[(int64_t)(q0 * CA_S + threadIdx.x) * gridDim.x + lb] = sum;
-  }
+    for (int t = 0; t < CA_S; ++t) v[c * CA_S + t] = (double)acc[c][t];
+  block_sums<CA_KQ * CA_S>(v, sh, nqt * CA_S, part + (int64_t)q0 * CA_S * gridDim.x + lb, gridDim.x);
 }
 
 // W[t] -= sum_q C[q][t] Q[q]  (C: nq x S, q-major), then partials of the Gram matrix of the
@@ -2709,7 +2736,7 @@ __global__ void __launch_bounds__(NTHR) k_bupdate_gram(int64_t n, const T *__res
                                                        double *__restrict__ part) {
   constexpr int VW = Vec<T>::w;
   __shared__ double cq[(CA_MMAX + 1) * CA_S];
-  __shared__ double sh[NTHR / 64][CA_NG];
+  __shared__ double sh[NTHR / 64][CA_NG + 1];
   for (int e = threadIdx.x; e < nq * CA_S; e += blockDim.x) cq[e] = C[e];
   __syncthreads();
   const int lb = xcd_block();
@@ -2774,18 +2801,11 @@ __global__ void __launch_bounds__(NTHR) k_bupdate_gram(int64_t n, const T *__res
       for (int a = 0; a < CA_S; ++a)
         for (int b = a; b < CA_S; ++b, ++g) gacc[g] += (double)o[a] * (double)o[b];
     }
+  double v[CA_NG + 1];  // (padded to an even number, which sums in fewer exchanges)
 #pragma unroll
-  for (int g = 0; g < CA_NG; ++g) {
-    const double v = wave_sum(gacc[g]);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][g] = v;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < CA_NG) {
-    double sum = 0.0;
-#pragma unroll
-    for (int wv = 0; wv < NTHR / 64; ++wv) sum += sh[wv][threadIdx.x];
-    part[(int64_t)threadIdx.x * gridDim.x + lb] = sum;
-  }
+  for (int g = 0; g < CA_NG; ++g) v[g] = gacc[g];
+  v[CA_NG] = 0.0;
+  block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, gridDim.x);
 }
 
 // W <- W Rinv (Rinv upper triangular S x S, row-major), Gram partials of the result if part
@@ -2794,7 +2814,7 @@ __global__ void __launch_bounds__(NTHR) k_btrsm_gram(int64_t n, T *__restrict__ 
                                                      const double *__restrict__ Rinv, double *__restrict__ part) {
   constexpr int VW = Vec<T>::w;
   __shared__ double ri[CA_S * CA_S];
-  __shared__ double sh[NTHR / 64][CA_NG];
+  __shared__ double sh[NTHR / 64][CA_NG + 1];
   if ((int)threadIdx.x < CA_S * CA_S) ri[threadIdx.x] = Rinv[threadIdx.x];
   __syncthreads();
   const int lb = xcd_block();
@@ -2849,18 +2869,11 @@ __global__ void __launch_bounds__(NTHR) k_btrsm_gram(int64_t n, T *__restrict__ 
       }
     }
   if (!part) return;
+  double v[CA_NG + 1];  // (padded to an even number, which sums in fewer exchanges)
 #pragma unroll
-  for (int g = 0; g < CA_NG; ++g) {
-    const double v = wave_sum(gacc[g]);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][g] = v;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < CA_NG) {
-    double sum = 0.0;
-#pragma unroll
-    for (int wv = 0; wv < NTHR / 64; ++wv) sum += sh[wv][threadIdx.x];
-    part[(int64_t)threadIdx.x * gridDim.x + lb] = sum;
-  }
+  for (int g = 0; g < CA_NG; ++g) v[g] = gacc[g];
+  v[CA_NG] = 0.0;
+  block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, gridDim.x);
 }
 
 // Cholesky G = R^T R of the packed Gram matrix; R and R^{-1} (row-major, upper). A non-positive
