@@ -2000,12 +2000,32 @@ static bool gather_supported(const Matrix *M, const std::vector<ocmp_term> &term
   return true;
 }
 
-// returns false (nothing launched) when some block pair needs more than 64 factors
-static bool launch_h1_gather(Matrix *M, const std::vector<ocmp_term> &vol, const std::vector<ocmp_field> &fields,
-                             bool accumulate) {
+// everything that a call's descriptors and tables are made from, by value
+static void plan_fields(std::string &key, const std::vector<ocmp_field> &fields) {
+  auto put = [&](const void *p, size_t n) { key.append((const char *)p, n); };
+  for (auto &f : fields) {
+    const Space &fs = f.space->s;
+    const Block &fb = fs.blocks[f.block];
+    const int v[5] = {fb.kind, fb.order, fs.nloc, fb.loc_off, fb.nloc};
+    put(v, sizeof v);
+    put(&fs.d_edofs.p, sizeof(void *));
+    put(&f.vec, sizeof(void *));
+  }
+}
+
+// The gather's factor sets, tables and descriptors for these terms, on the device; returns false when
+// some block pair needs more than 64 factors. Kept for the next call: a form is assembled with the
+// same terms again and again (only the contents of its fields change), and making the tables costs
+// host time (0.35 ms for 3D diffuse-interface Stokes, as long as its kernels on 48k tets).
+static bool gather_plan(Matrix *M, const std::vector<ocmp_term> &vol, const std::vector<ocmp_field> &fields,
+                        bool accumulate) {
+  std::string plan(1, accumulate ? '+' : '=');
+  for (auto &t : vol) plan.append((const char *)&t, sizeof t);
+  plan_fields(plan, fields);
+  if (M->gplan == plan) return true;
+  M->gplan.clear();
   Space &s = *M->space;
-  Ctx *ctx = M->ctx;
-  hipStream_t st = ctx->stream;
+  hipStream_t st = M->ctx->stream;
   const Mesh &m = *s.mesh;
   const int d = m.dim;
   OCMP_REQUIRE((int)vol.size() <= MAXTG && (int)fields.size() <= MAXF, "too many terms or fields in one call");
@@ -2148,8 +2168,22 @@ static bool launch_h1_gather(Matrix *M, const std::vector<ocmp_term> &vol, const
   std::memcpy(desc.data() + sizeof KF, &KG, sizeof KG);
   M->d_gdesc.alloc(desc.size());
   OCMP_HIP(hipMemcpyAsync(M->d_gdesc.p, desc.data(), desc.size(), hipMemcpyHostToDevice, st));
+  OCMP_HIP(hipStreamSynchronize(st));  // the copy reads host memory that goes out of scope
+  M->gplan_nf = NF;
+  M->gplan.swap(plan);
+  return true;
+}
+
+static bool launch_h1_gather(Matrix *M, const std::vector<ocmp_term> &vol, const std::vector<ocmp_field> &fields,
+                             bool accumulate) {
+  if (!gather_plan(M, vol, fields, accumulate)) return false;
+  Space &s = *M->space;
+  Ctx *ctx = M->ctx;
+  hipStream_t st = ctx->stream;
+  const Mesh &m = *s.mesh;
+  const int d = m.dim, NF = M->gplan_nf;
   const KFactors *dKF = reinterpret_cast<const KFactors *>(M->d_gdesc.p);
-  const KGather *dKG = reinterpret_cast<const KGather *>(M->d_gdesc.p + sizeof KF);
+  const KGather *dKG = reinterpret_cast<const KGather *>(M->d_gdesc.p + sizeof(KFactors));
   M->d_factors.alloc((size_t)m.nel * std::max(NF, 1));
   {
     KTimer tm(ctx, ctx->cls("assemble_h1_factors"), (double)m.nel * (8.0 * NF + 4.0 * (d + 1)) + 8.0 * m.nv * d);
@@ -2170,8 +2204,6 @@ static bool launch_h1_gather(Matrix *M, const std::vector<ocmp_term> &vol, const
     k_h1_gather<<<grid, 256, shm, st>>>(dKG, M->ngblk, M->d_gblk.p, M->d_pe.p, M->d_gunit.p, M->d_gend.p, M->d_gidx.p,
                                         M->d_factors.p, M->d_val.p);
   }
-  // the descriptor copy reads host memory that goes out of scope on return
-  OCMP_HIP(hipStreamSynchronize(st));
   OCMP_HIP(hipGetLastError());
   return true;
 }
@@ -2413,19 +2445,31 @@ static void ensure_dof_entries(Space &s) {
   std::swap(s.d_lptr.n, ptr.n);
 }
 
-void launch_assemble_linear(Space *sp, double *bvec, const std::vector<ocmp_lterm> &terms,
-                            const std::vector<ocmp_field> &fields, bool accumulate) {
-  Space &s = *sp;
-  Ctx *ctx = s.mesh->ctx;
-  hipStream_t st = ctx->stream;
+// a load vector's kernel arguments for these terms, kept for the next call with the same ones
+struct LinPlan {
+  KLArgs A;
+  bool has_dg = false, has_bnd = false, has_src = false;
+};
+constexpr size_t MAX_LIN_PLANS = 8;
+
+static LinPlan linear_plan(Space &s, const std::vector<ocmp_lterm> &terms, const std::vector<ocmp_field> &fields) {
+  std::string plan;
+  for (auto &t : terms) plan.append((const char *)&t, sizeof t);
+  plan_fields(plan, fields);
+  auto hit = s.lin_plans.find(plan);
+  if (hit != s.lin_plans.end()) {
+    LinPlan P;
+    std::memcpy(&P, hit->second.data(), sizeof P);
+    return P;
+  }
+  hipStream_t st = s.mesh->ctx->stream;
   const Mesh &m = *s.mesh;
   const int d = m.dim;
   OCMP_REQUIRE((int)terms.size() <= MAXT, "too many terms (max 8)");
   OCMP_REQUIRE((int)fields.size() <= MAXF, "too many fields (max 8)");
   OCMP_REQUIRE(s.nloc <= MAXL, "compound element has too many dofs");
-  bool all_l2 = true;
-  for (auto &b : s.blocks) all_l2 &= b.kind == OCMP_L2;
-  KLArgs A;
+  LinPlan P;
+  KLArgs &A = P.A;
   std::memset(&A, 0, sizeof A);
   TableBuilder tb;
   A.nterms = (int)terms.size();
@@ -2475,7 +2519,7 @@ void launch_assemble_linear(Space *sp, double *bvec, const std::vector<ocmp_lter
                  &gr[(size_t)q * fb.nloc * d]);
     kf.tab_phi = tb.add(phi);
   }
-  bool has_dg = false, has_bnd = false;
+  bool &has_dg = P.has_dg, &has_bnd = P.has_bnd;
   for (size_t i = 0; i < terms.size(); ++i) {
     const ocmp_lterm &t = terms[i];
     KLTerm &k = A.t[i];
@@ -2547,9 +2591,25 @@ void launch_assemble_linear(Space *sp, double *bvec, const std::vector<ocmp_lter
   for (auto &f : fields) key += "|f" + std::to_string((uintptr_t)f.space) + "," + std::to_string(f.block);
   DBuf<double> *tab = cached_table(s, key, tb, st);
   A.tab = tab->p;
+  for (auto &t : terms) P.has_src |= t.kind == OCMP_LFI_SOURCE;
+  if (s.lin_plans.size() >= MAX_LIN_PLANS) s.lin_plans.clear();
+  s.lin_plans[plan].assign((const char *)&P, sizeof P);
+  return P;
+}
+
+void launch_assemble_linear(Space *sp, double *bvec, const std::vector<ocmp_lterm> &terms,
+                            const std::vector<ocmp_field> &fields, bool accumulate) {
+  Space &s = *sp;
+  Ctx *ctx = s.mesh->ctx;
+  hipStream_t st = ctx->stream;
+  const Mesh &m = *s.mesh;
+  const int d = m.dim;
+  bool all_l2 = true;
+  for (auto &b : s.blocks) all_l2 &= b.kind == OCMP_L2;
+  const LinPlan P = linear_plan(s, terms, fields);
+  const KLArgs &A = P.A;
+  const bool has_dg = P.has_dg, has_bnd = P.has_bnd, has_src = P.has_src;
   KTimer tm(ctx, ctx->cls("assemble_linear"));
-  bool has_src = false;
-  for (auto &t : terms) has_src |= t.kind == OCMP_LFI_SOURCE;
   auto run = [&](double *out, int mode) {
     // 64 elements per workgroup of four wavefronts
     const unsigned gs = nblk(m.nel, 64), gf = nblk(m.nel * s.nloc);

@@ -191,6 +191,7 @@ struct Space {
   DBuf<uint32_t> d_lptr;  // ndof+1
   DBuf<uint32_t> d_lent;  // nel*nloc
   DBuf<double> d_lin;     // nloc*nel
+  std::map<std::string, std::string> lin_plans;  // load vectors: kernel arguments by terms and fields
   // cached kernel tables keyed by a signature
   std::map<std::string, DBuf<double> *> tables;
   ~Space() {
@@ -285,7 +286,9 @@ struct Matrix {
   int gemax = 0;
   DBuf<double> d_factors;            // nel x (factors per element) of the last assembly
   DBuf<int32_t> d_dslot;             // n: CSR slot of the diagonal entry (-1: none), built on first use
-  DBuf<char> d_gdesc;                // the gather's kernel descriptors
+  DBuf<char> d_gdesc;                // the gather's kernel descriptors for
+  std::string gplan;                 // these terms and fields (by value), with
+  int gplan_nf = 0;                  // so many factors per element
   // DG: per element-facet block position in the block row (0..3), diag block position
   DBuf<int8_t> d_dg_pos;             // nel*(dim+2): pos of diag block, then of each facet neighbour (-1 none)
   DBuf<int32_t> d_dg_bcol;           // nel*4 block columns (-1 padded), sorted
