@@ -271,67 +271,83 @@ __device__ __forceinline__ void load_run(const T *__restrict__ p, T (&v)[N]) {
   for (int i = 0; i < N; ++i) v[i] = u.t[i];
 }
 
-// One row block of a CSR product: xl(c) gives the (scaled) x value at column c, ef(r, s) receives each
-// row's sum, always in the same order of additions. Sums in the vector type (FP32 products in FP32,
-// FP64 in FP64).
-template <typename VT, typename XT, int NNZB, int NT, typename XL, typename EF>
-__device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, RbLds<XT, NNZB, NT> &S, XL xl, EF ef) {
+// What a thread loads for one row block before anything is computed: its run of nonzeros, its rows'
+// bounds, and the operands of x (raw values: xl) at four of the block's distinct columns, all of them
+// in blocks of 512 threads. None of it depends on scalars, so a kernel that first sums partial sums
+// has these loads in flight meanwhile.
+template <typename VT, int NNZB, int NT, typename RX>
+struct RbRegs {
+  RbDesc D;
+  VT v[NNZB / NT];
+  uint16_t li[NNZB / NT];
+  int ra[RB_ROWS / NT], re[RB_ROWS / NT];
+  RX x[4];
+};
+
+template <typename VT, int NNZB, int NT, typename RX, typename XL>
+__device__ __forceinline__ void rb_load(const RbCsr<VT> &M, const RbDesc &desc, RbRegs<VT, NNZB, NT, RX> &R, XL xl) {
   constexpr int PER = NNZB / NT;
   static_assert(PER % RB_ALIGN == 0 && PER <= 32, "runs are aligned and fit the mask");
+  const int tid = threadIdx.x;
+  R.D = desc;
+  const RbDesc &D = R.D;
+  if (D.kind == RB_LONG_ROW) return;
+  const int jb = D.j0 & ~(RB_ALIGN - 1);  // where the runs start
+  if (tid * PER < D.j0 - jb + D.nz) {
+    load_run<PER>(M.val + jb + tid * PER, R.v);
+    load_run<PER>(M.lcol + jb + tid * PER, R.li);
+  }
+#pragma unroll
+  for (int k = 0; k < RB_ROWS / NT; ++k) {
+    const int ri = min(tid + k * NT, D.nrows - 1);
+    R.ra[k] = M.rp[D.r0 + ri] - jb;
+    R.re[k] = M.rp[D.r0 + ri + 1] - jb;
+  }
+  // (indices past nu are clamped so that the gathers are unconditional)
+  if (D.nu > 0) {
+    int32_t c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = M.ucol[D.u0 + min(k * NT + tid, D.nu - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) R.x[k] = xl(c[k]);
+  }
+}
+
+// One row block of a CSR product: xf(xl(c)) is the x value at column c, ef(k, r, s) receives each row's sum
+// (r is the thread's k-th row, D.r0 + threadIdx.x + k NT, or k = -1), always in the same order of
+// additions. Sums in the vector type (FP32 products in FP32, FP64 in FP64).
+template <typename VT, typename XT, int NNZB, int NT, typename RX, typename XL, typename XF, typename EF>
+__device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, NT, RX> &R,
+                                           RbLds<XT, NNZB, NT> &S, XL xl, XF xf, EF ef) {
+  constexpr int PER = NNZB / NT;
   constexpr int RPT = RB_ROWS / NT;  // rows per thread
-  const RbDesc D = M.desc[lb];
+  const RbDesc &D = R.D;
   const int tid = threadIdx.x;
   if (D.kind == RB_LONG_ROW) {
     double s = 0.0;
-    for (int t = tid; t < D.nz; t += NT) {
-      const int32_t c = M.col[D.j0 + t];
-      s += (double)((XT)M.val[D.j0 + t] * xl(c));
-    }
+    for (int t = tid; t < D.nz; t += NT) s += (double)((XT)M.val[D.j0 + t] * xf(xl(M.col[D.j0 + t])));
     s = block_sum(s, S.red);
-    if (tid == 0) ef((int64_t)D.r0, s);
+    if (tid == 0) ef(-1, (int64_t)D.r0, s);
     return;
   }
-  const int jb = D.j0 & ~(RB_ALIGN - 1);  // where the runs start
-  const int d = D.j0 - jb, end = d + D.nz;
+  const int d = D.j0 & (RB_ALIGN - 1), end = d + D.nz;  // the block's part of the runs
   const int p0 = tid * PER;
-  VT v[PER];
-  uint16_t li[PER];
   const bool active = p0 < end;
-  if (active) {
-    load_run<PER>(M.val + jb + p0, v);
-    load_run<PER>(M.lcol + jb + p0, li);
-  }
-  int ra[RPT], re[RPT];
-#pragma unroll
-  for (int k = 0; k < RPT; ++k) {
-    const int ri = min(tid + k * NT, D.nrows - 1);
-    ra[k] = M.rp[D.r0 + ri] - jb;
-    re[k] = M.rp[D.r0 + ri + 1] - jb;
-  }
   S.ends[tid] = 0u;
   __syncthreads();
-  // x at the distinct columns (indices past nu are clamped so that a round's gathers are unconditional)
-  for (int base = 0; base < D.nu; base += 4 * NT) {
-    int32_t c[4];
+  // x at the distinct columns
 #pragma unroll
-    for (int k = 0; k < 4; ++k) c[k] = M.ucol[D.u0 + min(base + k * NT + tid, D.nu - 1)];
-    XT x[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) x[k] = xl(c[k]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int t = base + k * NT + tid;
-      if (t < D.nu) S.xs[t] = x[k];
-    }
-  }
+  for (int k = 0; k < 4; ++k)
+    if (k * NT + tid < D.nu) S.xs[k * NT + tid] = xf(R.x[k]);
+  for (int t = 4 * NT + tid; t < D.nu; t += NT) S.xs[t] = xf(xl(M.ucol[D.u0 + t]));
   if (D.kind == RB_PLAIN) {
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
       const int ri = tid + k * NT;
       if (ri < D.nrows) {
-        atomicOr(&S.ends[(re[k] - 1) / PER], 1u << ((re[k] - 1) % PER));
+        atomicOr(&S.ends[(R.re[k] - 1) / PER], 1u << ((R.re[k] - 1) % PER));
         // the runs whose first nonzero is in this row (row 0 also has the run that starts before it)
-        for (int t = ri == 0 ? 0 : (ra[k] + PER - 1) / PER; t * PER < re[k]; ++t) S.row[t] = (uint16_t)ri;
+        for (int t = ri == 0 ? 0 : (R.ra[k] + PER - 1) / PER; t * PER < R.re[k]; ++t) S.row[t] = (uint16_t)ri;
       }
     }
     __syncthreads();
@@ -340,19 +356,19 @@ __device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, Rb
 #pragma unroll
         for (int k = 0; k < PER; ++k)
           if (p0 + k < d || p0 + k >= end) {
-            v[k] = (VT)0;
-            li[k] = 0;
+            R.v[k] = (VT)0;
+            R.li[k] = 0;
           }
       }
       XT xv[PER];
 #pragma unroll
-      for (int k = 0; k < PER; ++k) xv[k] = S.xs[li[k]];
+      for (int k = 0; k < PER; ++k) xv[k] = S.xs[R.li[k]];
       const unsigned m = S.ends[tid];
       int row = S.row[tid];
       XT s = (XT)0;
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
-        s += (XT)v[k] * xv[k];
+        s += (XT)R.v[k] * xv[k];
         if (m >> k & 1u) {
           S.fin[row++] = s;
           s = (XT)0;
@@ -366,10 +382,10 @@ __device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, Rb
       const int ri = tid + k * NT;
       if (ri < D.nrows) {
         XT s = (XT)0;
-        const int tb = (re[k] - 1) / PER;
-        for (int t = ra[k] / PER; t < tb; ++t) s += S.car[t];
+        const int tb = (R.re[k] - 1) / PER;
+        for (int t = R.ra[k] / PER; t < tb; ++t) s += S.car[t];
         s += S.fin[ri];
-        ef((int64_t)(D.r0 + ri), (double)s);
+        ef(k, (int64_t)(D.r0 + ri), (double)s);
       }
     }
   } else {
@@ -378,9 +394,17 @@ __device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, Rb
     for (int ri = tid; ri < D.nrows; ri += NT) {
       XT s = (XT)0;
       for (int32_t j = M.rp[D.r0 + ri]; j < M.rp[D.r0 + ri + 1]; ++j) s += (XT)M.val[j] * S.xs[M.lcol[j]];
-      ef((int64_t)(D.r0 + ri), (double)s);
+      ef(-1, (int64_t)(D.r0 + ri), (double)s);
     }
   }
+}
+
+// the row block in one go: xl(c) gives the x value at column c, ef(r, s) receives each row's sum
+template <typename VT, typename XT, int NNZB, int NT, typename XL, typename EF>
+__device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, RbLds<XT, NNZB, NT> &S, XL xl, EF ef) {
+  RbRegs<VT, NNZB, NT, XT> R;
+  rb_load<VT, NNZB, NT, XT>(M, M.desc[lb], R, xl);
+  rb_compute<VT, XT, NNZB, NT, XT>(M, R, S, xl, [](XT x) { return x; }, [&](int, int64_t r, double s) { ef(r, s); });
 }
 
 template <typename VT, typename XT, int NNZB, int NT>
@@ -1078,6 +1102,13 @@ __global__ void __launch_bounds__(NTHR) k_cg_spmv(RbCsr<VT> M, const T *__restri
                                                   double *__restrict__ pqpart) {
   __shared__ RbLds<T, SPMV_NNZB, NTHR> lds;
   const bool first = it == 0;
+  const int lb = xcd_block();
+  struct Raw {
+    T z, p;
+  };
+  auto raw = [&](int64_t c) { return Raw{z[c], first ? (T)0 : pin[c]}; };
+  RbRegs<VT, SPMV_NNZB, NTHR, Raw> R;
+  if (lb < M.nrblk) rb_load<VT, SPMV_NNZB, NTHR, Raw>(M, M.desc[lb], R, raw);
   T beta = (T)0;
   if (!first) {
     double rz, rr;
@@ -1088,18 +1119,15 @@ __global__ void __launch_bounds__(NTHR) k_cg_spmv(RbCsr<VT> M, const T *__restri
       if (hist) hist[0] = rr;
     }
   }
-  const int lb = xcd_block();
   double acc = 0.0;
-  auto pnew = [&](int64_t c) { return first ? z[c] : z[c] + beta * pin[c]; };
+  auto pnew = [&](const Raw &w) { return w.z + beta * w.p; };
   if (lb < M.nrblk)
-    csr_row_block<VT, T, SPMV_NNZB, NTHR>(
-        M, lb, lds, [&](int32_t c) { return pnew(c); },
-        [&](int64_t r, double s) {
-          const T pr = pnew(r), v = mask[r] ? (T)s : (T)0;
-          pout[r] = pr;
-          q[r] = v;
-          acc += (double)pr * (double)v;
-        });
+    rb_compute<VT, T, SPMV_NNZB, NTHR, Raw>(M, R, lds, raw, pnew, [&](int, int64_t r, double s) {
+      const T pr = pnew(raw(r)), v = mask[r] ? (T)s : (T)0;
+      pout[r] = pr;
+      q[r] = v;
+      acc += (double)pr * (double)v;
+    });
   __syncthreads();
   acc = block_sum(acc, lds.red);
   if (threadIdx.x == 0) pqpart[lb] = acc;
@@ -3303,21 +3331,6 @@ __global__ void __launch_bounds__(NTHR) k_scg_init(int64_t n, const T *__restric
 // s_{i-1} (pointwise, by the same inline code as the owner); r, s and w are double-buffered by
 // iteration parity, so every value a block reads was written by an earlier launch. u is never
 // stored and p, x are only touched by their owner. u_0 = dinv r_0 (it = 0: beta = 0, no s_{-1}).
-template <typename T>
-struct ScgNext {
-  T s, r, u;
-};
-template <typename T>
-__device__ __forceinline__ ScgNext<T> scg_next(const T *__restrict__ rin, const T *__restrict__ win,
-                                               const T *__restrict__ sin, const T *__restrict__ dinv, int64_t c,
-                                               T a, T b, bool first) {
-  ScgNext<T> o;
-  o.s = first ? win[c] : win[c] + b * sin[c];
-  o.r = rin[c] - a * o.s;
-  o.u = dinv[c] * o.r;
-  return o;
-}
-
 template <typename T, typename VT, int NNZB, int NT>
 __global__ void __launch_bounds__(NT) k_scg_fused(
     RbCsr<VT> M, int it, double tol2, T *__restrict__ x, T *__restrict__ p, const T *__restrict__ rin,
@@ -3327,10 +3340,33 @@ __global__ void __launch_bounds__(NT) k_scg_fused(
     double *__restrict__ sc, int *__restrict__ flag) {
   __shared__ RbLds<T, NNZB, NT> lds;
   double *sh = lds.red;
-  if (*flag) return;
+  const bool first = it == 0;
+  const int lb = xcd_block();
+  // the vectors' values at a column, and of p and x at a row, loaded before the scalars are known
+  struct Raw {
+    T r, w, s, dinv;
+  };
+  auto raw = [&](int64_t c) { return Raw{rin[c], win[c], first ? (T)0 : sin[c], dinv[c]}; };
+  RbRegs<VT, NNZB, NT, Raw> R;
+  constexpr int RPT = RB_ROWS / NT;
+  Raw rv[RPT];
+  T pv[RPT], xv[RPT];
+  auto load = [&](const RbDesc &D) {
+    rb_load<VT, NNZB, NT, Raw>(M, D, R, raw);
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int64_t row = R.D.r0 + min((int)threadIdx.x + k * NT, R.D.nrows - 1);
+      rv[k] = raw(row);
+      pv[k] = first ? (T)0 : p[row];
+      xv[k] = x[row];
+    }
+  };
+  const RbDesc D0 = M.desc[min((int64_t)lb, M.nrblk - 1)];
+  if (*flag) return;  // (read along with the descriptor, which everything else waits for)
+  if (lb < M.nrblk) load(D0);
   double g, d;
   sum_parts2(gin, ng, din, nd, sh, g, d);
-  const double g0 = it == 0 ? g : sc[4];
+  const double g0 = first ? g : sc[4];
   if (!(g > tol2 * g0)) {  // converged (or a zero right-hand side): the same decision in every block
     if (blockIdx.x == 0 && threadIdx.x == 0) flag[0] = 1;
     return;
@@ -3349,29 +3385,41 @@ __global__ void __launch_bounds__(NT) k_scg_fused(
     sc[5] += 1.0;
   }
   const T a = (T)alpha, b = (T)beta;
-  const bool first = it == 0;
-  const int lb = xcd_block();
   double ag = 0.0, ad = 0.0;
-  // the owner's update of row k, given its new S u value
-  auto finish = [&](int64_t k, double sv) {
-    const ScgNext<T> o = scg_next<T>(rin, win, sin, dinv, k, a, b, first);
-    const T uo = dinv[k] * rin[k];
-    const T pk = first ? uo : uo + b * p[k];
-    p[k] = pk;
-    sout[k] = o.s;
-    x[k] += a * pk;
-    rout[k] = o.r;
+  // s_i, r_{i+1}, u_{i+1} from the loaded values, by the owner and by every block that needs u_{i+1}
+  struct Next {
+    T s, r, u;
+  };
+  auto next = [&](const Raw &v) {
+    Next o;
+    o.s = v.w + b * v.s;
+    o.r = v.r - a * o.s;
+    o.u = v.dinv * o.r;
+    return o;
+  };
+  // the owner's update of a row, given its new S u value
+  auto finish = [&](int k, int64_t row, double sv) {
+    const Raw v = k < 0 ? raw(row) : rv[k < 0 ? 0 : k];
+    const T pk = v.dinv * v.r + b * (k < 0 ? (first ? (T)0 : p[row]) : pv[k < 0 ? 0 : k]);
+    const T xk = k < 0 ? x[row] : xv[k < 0 ? 0 : k];
+    const Next o = next(v);
+    p[row] = pk;
+    sout[row] = o.s;
+    x[row] = xk + a * pk;
+    rout[row] = o.r;
     const T wk = (T)sv;
-    wout[k] = wk;
+    wout[row] = wk;
     ag += (double)o.r * (double)o.u;
     ad += (double)wk * (double)o.u;
   };
   // a grid of at most SCG_MAX_GRID blocks walks all row blocks, so the partials every block sums
   // stay few however large the matrix is
   for (int64_t rbk = lb; rbk < M.nrblk; rbk += gridDim.x) {
-    __syncthreads();  // the last row block's sums have been read
-    csr_row_block<VT, T, NNZB, NT>(
-        M, rbk, lds, [&](int32_t c) { return scg_next<T>(rin, win, sin, dinv, c, a, b, first).u; }, finish);
+    if (rbk != lb) {
+      load(M.desc[rbk]);
+      __syncthreads();  // the last row block's sums have been read
+    }
+    rb_compute<VT, T, NNZB, NT, Raw>(M, R, lds, raw, [&](const Raw &v) { return next(v).u; }, finish);
   }
   __syncthreads();
   ag = block_sum(ag, sh);
