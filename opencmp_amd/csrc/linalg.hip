@@ -401,10 +401,16 @@ __device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, 
 
 // the row block in one go: xl(c) gives the x value at column c, ef(r, s) receives each row's sum
 template <typename VT, typename XT, int NNZB, int NT, typename XL, typename EF>
-__device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, int64_t lb, RbLds<XT, NNZB, NT> &S, XL xl, EF ef) {
+__device__ __forceinline__ void csr_row_block(const RbCsr<VT> &M, const RbDesc &desc, RbLds<XT, NNZB, NT> &S, XL xl, EF ef) {
   RbRegs<VT, NNZB, NT, XT> R;
-  rb_load<VT, NNZB, NT, XT>(M, M.desc[lb], R, xl);
+  rb_load<VT, NNZB, NT, XT>(M, desc, R, xl);
   rb_compute<VT, XT, NNZB, NT, XT>(M, R, S, xl, [](XT x) { return x; }, [&](int, int64_t r, double s) { ef(r, s); });
+}
+// a block's descriptor (the last one's for blocks past the end), read before the flag that may end the
+// launch so that the two loads overlap
+template <typename T>
+__device__ __forceinline__ RbDesc rb_desc(const RbCsr<T> &M, int64_t lb) {
+  return M.desc[min(lb, M.nrblk - 1)];
 }
 
 template <typename VT, typename XT, int NNZB, int NT>
@@ -414,14 +420,15 @@ __global__ void __launch_bounds__(NT) k_spmv_csr(RbCsr<VT> M, const XT *__restri
                                                    double *__restrict__ part, XT dsh, const XT *__restrict__ xp,
                                                    XT csh, const int *__restrict__ skip,
                                                    const int32_t *__restrict__ rowmap) {
-  if (skip && *skip) return;  // a converged inner solve: the rest of its fixed launch sequence is empty
   __shared__ RbLds<XT, NNZB, NT> lds;
   const int lb = xcd_block();
+  const RbDesc desc = rb_desc(M, lb);
+  if (skip && *skip) return;  // a converged inner solve: the rest of its fixed launch sequence is empty
   double acc = 0.0;
   const XT scale = (mode == 3 && sx) ? (XT)sx[0] : (XT)1;
   if (lb < M.nrblk)
     csr_row_block<VT, XT, NNZB, NT>(
-        M, lb, lds,
+        M, desc, lds,
         [&](int32_t c) { return (mode >= 3 && cs) ? x[c] * cs[c] : x[c]; },
         [&](int64_t r, double s) {
           // a reordered operator's row r is row rowmap[r] of the vectors
@@ -1035,6 +1042,13 @@ __global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x
                                                     const double *__restrict__ pqpart, int npq,
                                                     double *__restrict__ part) {
   __shared__ double sh[2 * NTHR / 64];
+  const double rz0 = sc[it & 1];
+  const int lb = xcd_block();
+  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
+  const int64_t i0 = lb * chunk, i1 = min(n, i0 + chunk);
+  // the first element's operands, loaded while the scalars are on their way
+  const int64_t f = min(i0 + (int64_t)threadIdx.x, n - 1);
+  const T rf = r[f], qf = q[f], df = dinv[f], pf = x ? p[f] : (T)0, xf = x ? x[f] : (T)0;
   double pq;
   if (npq > 0) {
     double none;
@@ -1043,16 +1057,14 @@ __global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x
   } else {
     pq = sc[2];
   }
-  const T alpha = (T)(sc[it & 1] / pq);
-  const int lb = xcd_block();
-  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-  const int64_t i0 = lb * chunk, i1 = min(n, i0 + chunk);
+  const T alpha = (T)(rz0 / pq);
   double rz = 0.0, rr = 0.0;
   for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    if (x) x[i] += alpha * p[i];
-    const T ri = r[i] - alpha * q[i];
+    const bool one = i == f;
+    if (x) x[i] = (one ? xf : x[i]) + alpha * (one ? pf : p[i]);
+    const T ri = (one ? rf : r[i]) - alpha * (one ? qf : q[i]);
     r[i] = ri;
-    const T zi = dinv[i] * ri;
+    const T zi = (one ? df : dinv[i]) * ri;
     z[i] = zi;
     rz += (double)ri * (double)zi;
     rr += (double)ri * (double)ri;
@@ -1108,12 +1120,24 @@ __global__ void __launch_bounds__(NTHR) k_cg_spmv(RbCsr<VT> M, const T *__restri
   };
   auto raw = [&](int64_t c) { return Raw{z[c], first ? (T)0 : pin[c]}; };
   RbRegs<VT, SPMV_NNZB, NTHR, Raw> R;
-  if (lb < M.nrblk) rb_load<VT, SPMV_NNZB, NTHR, Raw>(M, M.desc[lb], R, raw);
+  constexpr int RPT = RB_ROWS / NTHR;
+  Raw rv[RPT];
+  uint8_t mv[RPT];
+  const double old = sc[(it + 1) & 1];
+  if (lb < M.nrblk) {
+    rb_load<VT, SPMV_NNZB, NTHR, Raw>(M, M.desc[lb], R, raw);
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int64_t row = R.D.r0 + min((int)threadIdx.x + k * NTHR, R.D.nrows - 1);
+      rv[k] = raw(row);
+      mv[k] = mask[row];
+    }
+  }
   T beta = (T)0;
   if (!first) {
     double rz, rr;
     sum_parts2(part, np, part + np, np, lds.red, rz, rr);
-    beta = (T)(rz / sc[(it + 1) & 1]);
+    beta = (T)(rz / old);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       sc[it & 1] = rz;
       if (hist) hist[0] = rr;
@@ -1122,8 +1146,9 @@ __global__ void __launch_bounds__(NTHR) k_cg_spmv(RbCsr<VT> M, const T *__restri
   double acc = 0.0;
   auto pnew = [&](const Raw &w) { return w.z + beta * w.p; };
   if (lb < M.nrblk)
-    rb_compute<VT, T, SPMV_NNZB, NTHR, Raw>(M, R, lds, raw, pnew, [&](int, int64_t r, double s) {
-      const T pr = pnew(raw(r)), v = mask[r] ? (T)s : (T)0;
+    rb_compute<VT, T, SPMV_NNZB, NTHR, Raw>(M, R, lds, raw, pnew, [&](int k, int64_t r, double s) {
+      const T pr = pnew(k < 0 ? raw(r) : rv[k < 0 ? 0 : k]);
+      const T v = (k < 0 ? mask[r] : mv[k < 0 ? 0 : k]) ? (T)s : (T)0;
       pout[r] = pr;
       q[r] = v;
       acc += (double)pr * (double)v;
@@ -1296,13 +1321,14 @@ __device__ void givens_step(const GState &G, int j, double hn) {
     __syncthreads();
   }
   if (threadIdx.x == 0) {
+    // (the entry that the rotations carry down stays in a register)
+    double a = col[0];
     for (int k = 0; k < j; ++k) {
-      const double c = rot[2 * k], s = rot[2 * k + 1];
-      const double a = col[k], b = col[k + 1];
+      const double c = rot[2 * k], s = rot[2 * k + 1], b = col[k + 1];
       col[k] = c * a + s * b;
-      col[k + 1] = -s * a + c * b;
+      a = -s * a + c * b;
     }
-    const double a = col[j], b = col[j + 1];
+    const double b = hn;
     const double den = hypot(a, b);
     const double c = den > 0.0 ? a / den : 1.0, s = den > 0.0 ? b / den : 0.0;
     G.csn[2 * j] = c;
@@ -1376,9 +1402,9 @@ __global__ void __launch_bounds__(NTHR) k_gs_update(int64_t n, const T *__restri
 __global__ void __launch_bounds__(256) k_norm_givens(const double *__restrict__ part, int nparts, int j, GState G) {
   __shared__ double sh[4];
   __shared__ double hn;
+  double s = (int)threadIdx.x < nparts ? part[threadIdx.x] : 0.0;
   if (G.done && *G.done) return;  // read by every thread before the first barrier; set only after it
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nparts; b += blockDim.x) s += part[b];
+  for (int b = threadIdx.x + blockDim.x; b < nparts; b += blockDim.x) s += part[b];
   s = block_sum(s, sh);
   if (threadIdx.x == 0) hn = sqrt(s);
   __syncthreads();
@@ -1390,9 +1416,32 @@ __global__ void __launch_bounds__(256) k_norm_givens(const double *__restrict__ 
 __global__ void __launch_bounds__(256) k_gmres_solve(int k, int m, const double *__restrict__ R,
                                                      const double *__restrict__ g, const double *__restrict__ vs,
                                                      double *__restrict__ coef) {
+  const int ld = m + 1;
+  if (k <= 64) {
+    // one wavefront, lane r with row r of the right-hand side: no barriers, eight columns' loads ahead
+    // of the steps that use them (50 columns: 9 us, 28-36 with a barrier and a load a step)
+    const int r = threadIdx.x;
+    if (r >= 64) return;
+    double y = r < k ? g[r] : 0.0;
+    const double dr = r < k ? R[(int64_t)r * ld + r] : 1.0;
+    for (int i0 = k - 1; i0 >= 0; i0 -= 8) {
+      double c[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c[u] = R[(int64_t)max(i0 - u, 0) * ld + min(r, max(i0 - u, 0))];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = i0 - u;
+        if (i < 0) break;
+        const double yi = __shfl(y / dr, i, 64);
+        if (r == i) y = yi;
+        else if (r < i) y -= c[u] * yi;
+      }
+    }
+    if (r < k) coef[r] = vs ? y * vs[r] : y;
+    return;
+  }
   __shared__ double gs[256];
   __shared__ double yi;
-  const int ld = m + 1;
   for (int i = threadIdx.x; i < k; i += blockDim.x) gs[i] = g[i];
   __syncthreads();
   for (int i = k - 1; i >= 0; --i) {
@@ -1804,8 +1853,9 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
                                                    T w, T *__restrict__ z, T *__restrict__ bc, T *__restrict__ bout,
                                                    JacRows<T> J, const int *__restrict__ skip) {
   __shared__ RbLds<T, NNZB, NTHR> lds;
-  if (skip && *skip) return;  // a converged FGMRES cycle: its remaining launches are empty
   const int lb = xcd_block();
+  const RbDesc desc = lb < ga ? rb_desc(A, lb) : rb_desc(Wt, lb - ga);
+  if (skip && *skip) return;  // a converged FGMRES cycle: its remaining launches are empty
   const double g = sig ? -sig[0] : 1.0;
   const int gw = (int)gridDim.x - ga - J.nblk;  // blocks of the W^T task
   if (lb >= ga + gw) {
@@ -1817,7 +1867,7 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
   if (lb < ga) {
     if (lb >= A.nrblk) return;
     csr_row_block<T, T, NNZB, NTHR>(
-        A, lb, lds, [&](int32_t c) { return u[c] * dinv[c]; },
+        A, desc, lds, [&](int32_t c) { return u[c] * dinv[c]; },
         [&](int64_t r, double s) {
           const double b = g * (double)u[r];
           z[r] = (T)((double)w * (double)dinv[r] * (2.0 * b - (double)w * g * s));
@@ -1827,7 +1877,7 @@ __global__ void __launch_bounds__(NTHR) k_amg_down(int ga, RbCsr<T> A, RbCsr<T> 
     const int wb = lb - ga;
     if (wb >= Wt.nrblk) return;
     csr_row_block<T, T, NNZB, NTHR>(
-        Wt, wb, lds, [&](int32_t c) { return u[c]; }, [&](int64_t r, double s) { bc[r] = (T)(g * s); });
+        Wt, desc, lds, [&](int32_t c) { return u[c]; }, [&](int64_t r, double s) { bc[r] = (T)(g * s); });
   }
 }
 
@@ -3661,8 +3711,9 @@ static int fgmres_cycle(Matrix *A, Matrix *K, Precond *P, bool learned, const do
   int j = 0, bidx = 0, k_used = -1;
   // inner solve (Schur PCG, or the velocity PCG of the block-triangular step) with a tolerance:
   // each step enqueues `cap` iterations (the rest of a converged inner solve are empty launches);
-  // after each batch the host reads how many ran and sets the cap to 1.3x that plus 10, doubling
-  // it when a step used them all
+  // after each batch the host reads how many ran and sets the cap to 1.1x that plus 4 (the count
+  // changes by a few from step to step: with 1.3x plus 10 half of the launches of a 3D diffuse-interface
+  // Stokes solve were empty, at 2.3 us each), doubling it when a step used them all
   const bool btri = P->btri;
   const int in_iters = btri ? P->vel_iters : P->schur_iters;
   const bool adapt = in_iters > 0 && (btri ? P->vel_tol : P->schur_tol) > 0.0;
@@ -3754,7 +3805,7 @@ static int fgmres_cycle(Matrix *A, Matrix *K, Precond *P, bool learned, const do
       const double cnt = hres[m + 2 + b.ev];
       const double per = (cnt - in_seen) / nb_run;
       in_seen = cnt;
-      in_cap = per >= b.cap - 0.5 ? std::min(in_iters, 2 * b.cap) : std::min(in_iters, (int)(1.3 * per) + 10);
+      in_cap = per >= b.cap - 0.5 ? std::min(in_iters, 2 * b.cap) : std::min(in_iters, (int)(1.1 * per) + 4);
     }
     if (conv >= 0) k_used = b.j0 + conv + 1;
   }
