@@ -44,11 +44,37 @@ __device__ __forceinline__ int xcd_block() {
   return (blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
 }
 
+// v's value in another lane of the row of 16 (row_shr:n) or from the previous rows (row_bcast:15, 31) by
+// data-parallel-primitive moves, 0 where there is none
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp0(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, ROWS == 0xf));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp0(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, ROWS == 0xf),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, ROWS == 0xf));
+}
+__device__ __forceinline__ float last_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+__device__ __forceinline__ double last_lane(double v) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// sum over the wave, in every lane. Moves between lanes of the vector unit instead of the LDS unit's
+// permutes, whose latency (six in a row, twice that for doubles) was a large part of the small
+// launches' time (one sum of 1024 partials 4.1 -> 3.1 us, the CG update of 4,225 rows 5.2 -> 4.4)
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+  v += dpp0<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8: lane 15 of a row has the row's sum
+  v += dpp0<0x112, 0xf>(v);
+  v += dpp0<0x114, 0xf>(v);
+  v += dpp0<0x118, 0xf>(v);
+  v += dpp0<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp0<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return last_lane(v);
 }
 
 // Sums of N values over the wave, several at a time: at each exchange a lane passes on one half of its
@@ -110,6 +136,25 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
   }
   __syncthreads();
   return s;
+}
+
+// the block's sums of two values, valid in thread 0; sh: two per wave
+__device__ __forceinline__ void block_sum2(double &a, double &b, double *sh) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  const int wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    sh[wid] = a;
+    sh[nw + wid] = b;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a = b = 0.0;
+    for (int i = 0; i < nw; ++i) {
+      a += sh[i];
+      b += sh[nw + i];
+    }
+  }
 }
 
 // 16-byte vector access
@@ -1069,8 +1114,7 @@ __global__ void __launch_bounds__(NTHR) k_cg_update(int64_t n, T *__restrict__ x
     rz += (double)ri * (double)zi;
     rr += (double)ri * (double)ri;
   }
-  rz = block_sum(rz, sh);
-  rr = block_sum(rr, sh);
+  block_sum2(rz, rr, sh);
   if (threadIdx.x == 0) {
     part[lb] = rz;
     part[gridDim.x + lb] = rr;
@@ -1938,15 +1982,30 @@ __global__ void __launch_bounds__(256) k_amg_tail_mv(int64_t n, int64_t ld, cons
                                                      const int *__restrict__ skip) {
   constexpr int VW = Vec<T>::w;
   __shared__ double bs[AMG_TAIL_LD];
+  const int lane = threadIdx.x & 63;
+  int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  // the first of the row's pieces, loaded while b is staged (pieces past its end are dropped below)
+  T a0[4][VW];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    vload(M + min(i, n - 1) * ld + min((int64_t)(lane + 64 * u) * VW, ld - VW), a0[u]);
   if (skip && *skip) return;
   for (int64_t j = threadIdx.x; j < ld; j += blockDim.x) bs[j] = j < n ? (double)b[j] : 0.0;
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += (int64_t)gridDim.x * 4) {
+  for (bool first = true; i < n; i += (int64_t)gridDim.x * 4, first = false) {
     const T *row = M + i * ld;
     double s = 0.0;
+    int64_t j = (int64_t)lane * VW;
+    if (first) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u, j += 64 * VW)
+        if (j < ld) {
+#pragma unroll
+          for (int l = 0; l < VW; ++l) s += (double)a0[u][l] * bs[j + l];
+        }
+    }
 #pragma unroll 4
-    for (int64_t j = (int64_t)lane * VW; j < ld; j += 64 * VW) {
+    for (; j < ld; j += 64 * VW) {
       T a[VW];
       vload(row + j, a);
 #pragma unroll
@@ -3412,18 +3471,18 @@ __global__ void __launch_bounds__(NT) k_scg_fused(
     }
   };
   const RbDesc D0 = M.desc[min((int64_t)lb, M.nrblk - 1)];
+  const double s4 = sc[4], gp = sc[2 * ((it + 1) & 1)], ap = sc[2 * ((it + 1) & 1) + 1];
   if (*flag) return;  // (read along with the descriptor, which everything else waits for)
   if (lb < M.nrblk) load(D0);
   double g, d;
   sum_parts2(gin, ng, din, nd, sh, g, d);
-  const double g0 = first ? g : sc[4];
+  const double g0 = first ? g : s4;
   if (!(g > tol2 * g0)) {  // converged (or a zero right-hand side): the same decision in every block
     if (blockIdx.x == 0 && threadIdx.x == 0) flag[0] = 1;
     return;
   }
   double beta = 0.0, den = d;
   if (it > 0) {
-    const double gp = sc[2 * ((it + 1) & 1)], ap = sc[2 * ((it + 1) & 1) + 1];
     beta = gp != 0.0 ? g / gp : 0.0;
     if (ap != 0.0) den = d - beta * g / ap;
   }
@@ -3472,8 +3531,7 @@ __global__ void __launch_bounds__(NT) k_scg_fused(
     rb_compute<VT, T, NNZB, NT, Raw>(M, R, lds, raw, [&](const Raw &v) { return next(v).u; }, finish);
   }
   __syncthreads();
-  ag = block_sum(ag, sh);
-  ad = block_sum(ad, sh);
+  block_sum2(ag, ad, sh);
   if (threadIdx.x == 0) {
     gout[lb] = ag;
     dout[lb] = ad;
