@@ -2781,6 +2781,7 @@ constexpr int CA_KQ_MAX = 16;
 // at condition ~1e4 instead of ~1e7 for plain powers (small enough for FP32 storage).
 constexpr double CA_SIGMA = 1.0;
 constexpr int CA_NG = CA_S * (CA_S + 1) / 2;
+constexpr int CA_FAC_BLOCKS = 1024;
 // largest restart of an s-step cycle: the block kernels size their LDS for k + 1 + CA_S <= CA_MMAX + 1
 // basis rows (the host only takes the s-step path for m <= CA_MMAX)
 constexpr int CA_MMAX = 50;
@@ -2899,7 +2900,21 @@ __global__ void __launch_bounds__(NTHR) k_bupdate_gram(int64_t n, const T *__res
 #pragma unroll
       for (int l = 0; l < VW; ++l) w[l][t] = (double)wv[t][l];
     }
-    for (int q = 0; q < nq; ++q) {
+    int q = 0;
+    for (; q + CA_S < nq; q += CA_S) {  // nq is 1 mod CA_S: whole blocks of rows, then one row
+      T qv[CA_S][VW];
+#pragma unroll
+      for (int r = 0; r < CA_S; ++r) vload(Q + (int64_t)(q + r) * ldv + i * VW, qv[r]);
+#pragma unroll
+      for (int r = 0; r < CA_S; ++r)
+#pragma unroll
+        for (int t = 0; t < CA_S; ++t) {
+          const double c = cq[(q + r) * CA_S + t];
+#pragma unroll
+          for (int l = 0; l < VW; ++l) w[l][t] -= c * (double)qv[r][l];
+        }
+    }
+    for (; q < nq; ++q) {
       T qv[VW];
       vload(Q + (int64_t)q * ldv + i * VW, qv);
 #pragma unroll
@@ -2945,87 +2960,16 @@ __global__ void __launch_bounds__(NTHR) k_bupdate_gram(int64_t n, const T *__res
   block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, gridDim.x);
 }
 
-// W <- W Rinv (Rinv upper triangular S x S, row-major), Gram partials of the result if part
-template <typename T>
-__global__ void __launch_bounds__(NTHR) k_btrsm_gram(int64_t n, T *__restrict__ W, int64_t ldv,
-                                                     const double *__restrict__ Rinv, double *__restrict__ part) {
-  constexpr int VW = Vec<T>::w;
-  __shared__ double ri[CA_S * CA_S];
-  __shared__ double sh[NTHR / 64][CA_NG + 1];
-  if ((int)threadIdx.x < CA_S * CA_S) ri[threadIdx.x] = Rinv[threadIdx.x];
-  __syncthreads();
-  const int lb = xcd_block();
-  const int64_t nvec = n / VW;
-  const int64_t chunk = (nvec + gridDim.x - 1) / gridDim.x;
-  const int64_t i0 = lb * chunk, i1 = min(nvec, i0 + chunk);
-  double gacc[CA_NG];
-#pragma unroll
-  for (int g = 0; g < CA_NG; ++g) gacc[g] = 0.0;
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    T wv[CA_S][VW];
-#pragma unroll
-    for (int t = 0; t < CA_S; ++t) vload(W + (int64_t)t * ldv + i * VW, wv[t]);
-    T ov[CA_S][VW];
-#pragma unroll
-    for (int l = 0; l < VW; ++l)
-#pragma unroll
-      for (int t = 0; t < CA_S; ++t) {
-        double sum = 0.0;
-#pragma unroll
-        for (int a = 0; a <= t; ++a) sum += (double)wv[a][l] * ri[a * CA_S + t];
-        ov[t][l] = (T)sum;
-      }
-#pragma unroll
-    for (int t = 0; t < CA_S; ++t) vstore(W + (int64_t)t * ldv + i * VW, ov[t]);
-    if (part) {
-#pragma unroll
-      for (int l = 0; l < VW; ++l) {
-        int g = 0;
-#pragma unroll
-        for (int a = 0; a < CA_S; ++a)
-#pragma unroll
-          for (int b = a; b < CA_S; ++b, ++g) gacc[g] += (double)ov[a][l] * (double)ov[b][l];
-      }
-    }
-  }
-  if (lb == gridDim.x - 1)
-    for (int64_t i = nvec * VW + threadIdx.x; i < n; i += blockDim.x) {
-      double w[CA_S];
-      T o[CA_S];
-      for (int t = 0; t < CA_S; ++t) w[t] = (double)W[(int64_t)t * ldv + i];
-      for (int t = 0; t < CA_S; ++t) {
-        double sum = 0.0;
-        for (int a = 0; a <= t; ++a) sum += w[a] * ri[a * CA_S + t];
-        o[t] = (T)sum;
-        W[(int64_t)t * ldv + i] = o[t];
-      }
-      if (part) {
-        int g = 0;
-        for (int a = 0; a < CA_S; ++a)
-          for (int b = a; b < CA_S; ++b, ++g) gacc[g] += (double)o[a] * (double)o[b];
-      }
-    }
-  if (!part) return;
-  double v[CA_NG + 1];  // (padded to an even number, which sums in fewer exchanges)
-#pragma unroll
-  for (int g = 0; g < CA_NG; ++g) v[g] = gacc[g];
-  v[CA_NG] = 0.0;
-  block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, gridDim.x);
-}
-
-// Cholesky G = R^T R of the packed Gram matrix; R and R^{-1} (row-major, upper). A non-positive
-// pivot sets *flag (the block is then discarded by the host) and returns the identity. Every loop
-// has a constant trip count so the 5x5 arrays stay in registers. ident, if given, is set to the
-// identity (the second factor of a single-pass CholQR).
-__global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R, double *__restrict__ Rinv,
-                          double *__restrict__ flag, double *__restrict__ ident) {
-  if (ident && threadIdx.x < CA_S * CA_S) ident[threadIdx.x] = (threadIdx.x / CA_S == threadIdx.x % CA_S) ? 1.0 : 0.0;
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Cholesky G = R^T R of the packed Gram matrix; R and R^{-1} (row-major, upper), by one thread. A
+// non-positive pivot returns false and the identity. Every loop has a constant trip count so the
+// 5x5 arrays stay in registers.
+__device__ __forceinline__ bool ca_cholesky(const double *gp, double *R, double *Rinv) {
   double G[CA_S][CA_S], U[CA_S][CA_S], Ui[CA_S][CA_S];
 #pragma unroll
   for (int a = 0; a < CA_S; ++a)
 #pragma unroll
     for (int b = a; b < CA_S; ++b) G[a][b] = G[b][a] = gp[a * CA_S - a * (a - 1) / 2 + (b - a)];
+  double ip[CA_S];  // reciprocal pivots: one division each in the chain
   bool ok = true;
 #pragma unroll
   for (int j = 0; j < CA_S; ++j) {
@@ -3034,6 +2978,7 @@ __global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R,
     for (int k = 0; k < j; ++k) d -= U[k][j] * U[k][j];
     ok = ok && d > 0.0;
     U[j][j] = sqrt(d > 0.0 ? d : 1.0);
+    ip[j] = 1.0 / U[j][j];
 #pragma unroll
     for (int c = 0; c < j; ++c) U[j][c] = 0.0;
 #pragma unroll
@@ -3041,17 +2986,16 @@ __global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R,
       double v = G[j][c];
 #pragma unroll
       for (int k = 0; k < j; ++k) v -= U[k][j] * U[k][c];
-      U[j][c] = v / U[j][j];
+      U[j][c] = v * ip[j];
     }
   }
   if (!ok) {
-    flag[0] = 1.0;
 #pragma unroll
     for (int i = 0; i < CA_S * CA_S; ++i) {
       R[i] = (i / CA_S == i % CA_S) ? 1.0 : 0.0;
       Rinv[i] = (i / CA_S == i % CA_S) ? 1.0 : 0.0;
     }
-    return;
+    return false;
   }
   // inverse of the upper triangular U, column by column (back substitution)
 #pragma unroll
@@ -3061,7 +3005,7 @@ __global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R,
       double v = (r == c) ? 1.0 : 0.0;
 #pragma unroll
       for (int k = r + 1; k < CA_S; ++k) v -= U[r][k] * Ui[k][c];
-      Ui[r][c] = v / U[r][r];
+      Ui[r][c] = v * ip[r];
     }
 #pragma unroll
   for (int a = 0; a < CA_S; ++a)
@@ -3070,6 +3014,45 @@ __global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R,
       R[a * CA_S + b] = U[a][b];
       Rinv[a * CA_S + b] = (b < a) ? 0.0 : Ui[a][b];
     }
+  return true;
+}
+
+// The Gram matrix from its np partials per entry, and its factors, by one block of NW waves: a wave
+// sums every NW-th entry. gs: CA_NG doubles, R and Ri: CA_S^2 each, all in LDS. *ok is valid for all
+// threads afterwards.
+template <int NW>
+__device__ __forceinline__ void ca_factor_block(const double *__restrict__ gpart, int np, double *gs, double *R,
+                                                double *Ri, int *ok) {
+  constexpr int U = (CA_NG + NW - 1) / NW;
+  const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
+  double s[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) s[u] = 0.0;
+  for (int b = ln; b < np; b += 64)
+#pragma unroll
+    for (int u = 0; u < U; ++u) s[u] += gpart[(int64_t)min(wv + u * NW, CA_NG - 1) * np + b];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const double t = wave_sum(s[u]);
+    if (ln == 0 && wv + u * NW < CA_NG) gs[wv + u * NW] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *ok = ca_cholesky(gs, R, Ri) ? 1 : 0;
+  __syncthreads();
+}
+
+// The Gram matrix' partials summed and factored in one launch of one block, a wave an entry (768 partials:
+// 6.1 us; a launch to sum and one to factor before: 4.5 + 4.2 us)
+__global__ void __launch_bounds__(1024) k_ca_chol(const double *__restrict__ gpart, int np, double *__restrict__ R,
+                                                  double *__restrict__ Rinv, double *__restrict__ flag) {
+  __shared__ double gs[CA_NG], Rl[CA_S * CA_S], Ri[CA_S * CA_S];
+  __shared__ int ok;
+  ca_factor_block<16>(gpart, np, gs, Rl, Ri, &ok);
+  if (threadIdx.x < CA_S * CA_S) {
+    R[threadIdx.x] = Rl[threadIdx.x];
+    Rinv[threadIdx.x] = Ri[threadIdx.x];
+  }
+  if (threadIdx.x == 0 && !ok) flag[0] = 1.0;
 }
 
 // New Hessenberg columns k..k+S-1 from the change of basis (Ahat v_t = v_{t+1} + d_t v_t -
@@ -3078,46 +3061,72 @@ __global__ void k_ca_chol(const double *__restrict__ gp, double *__restrict__ R,
 // The residual estimates of the new columns and the CholQR breakdown flag also go straight to the
 // host's pinned status buffer hst (res at [j], the flag at [m + 8 + slot]); the host reads them
 // after the event recorded behind this kernel.
-__global__ void __launch_bounds__(256) k_ca_hess(int k, int m, const double *__restrict__ C,
-                                                 const double *__restrict__ R1, const double *__restrict__ R2,
-                                                 double *__restrict__ Hf, GState G, CaShift B,
-                                                 const double *__restrict__ flag, double *__restrict__ hst,
-                                                 int slot) {
-  constexpr int MAXR = CA_MMAX + 1;  // rows of the basis: k + 1 + CA_S <= m + 1
-  __shared__ double Rr[MAXR * (CA_S + 1)];          // (k+1+S) x (S+1), column-major
-  __shared__ double HC[(CA_MMAX + 1) * CA_S];       // H_old (k+1 x k) @ Rr[0:k, 0:S]
-  __shared__ double Rt[CA_S * CA_S];
-  __shared__ double Hn[MAXR * CA_S];
-  __shared__ double rot[2 * MAXR];                  // the k rotations of the earlier columns
-  __shared__ double tl[CA_S][CA_S + 2];             // rows k..k+c+1 of column k+c after those rotations
-  const int ld = m + 1, nr = k + 1 + CA_S;
+struct CaHess {
+  int on, k, m, slot;
+  const double *C, *R1, *R2;  // R1, R2: the factors of the first and second pass; R2 is null after a single pass
+  double *Hf;
+  GState G;
+  CaShift B;
+  double *hst;
+};
+// The old columns' part of the new ones is a product with the whole of H_old: thread (row r, slice sl) holds
+// its CA_HT entries from before the factor is known.
+constexpr int CA_MAXR = CA_MMAX + 1;  // rows of the basis: k + 1 + CA_S <= m + 1
+constexpr int CA_HT = (CA_MMAX - CA_S + CA_S - 1) / CA_S;
+static_assert(CA_MAXR * CA_S <= NTHR, "a thread per row and slice of the old columns");
+struct CaHessLds {
+  double Rr[CA_MAXR * (CA_S + 1)];    // (k+1+S) x (S+1), column-major: the block in terms of the basis
+  double hp[CA_S][CA_S][CA_MAXR];     // partial sums over a slice of H_old (k+1 x k) @ Rr[0:k, 0:S]
+  double Hn[CA_MAXR * CA_S];
+  double rot[2 * CA_MAXR];            // the k rotations of the earlier columns
+  double tl[CA_S][CA_S + 2];          // rows k..k+c+1 of column k+c after those rotations
+};
+__device__ __forceinline__ void ca_hess_load(const CaHess &h, CaHessLds &l, double (&hr)[CA_HT]) {
+  const int k = h.k, ld = h.m + 1, nr = k + 1 + CA_S, tid = threadIdx.x;
+  const int r = tid % CA_MAXR, sl = tid / CA_MAXR;
+#pragma unroll
+  for (int j = 0; j < CA_HT; ++j) {
+    const int t = sl * CA_HT + j;
+    hr[j] = t < k && r <= t + 1 ? h.Hf[(int64_t)t * ld + r] : 0.0;  // H_old is upper Hessenberg
+  }
+  for (int e = tid; e < 2 * k; e += blockDim.x) l.rot[e] = h.G.csn[e];
+  for (int e = tid; e < (k + 1) * CA_S; e += blockDim.x) l.Rr[(e % CA_S + 1) * nr + e / CA_S] = h.C[e];
+  for (int e = tid; e < nr; e += blockDim.x) l.Rr[e] = e == k ? 1.0 : 0.0;
+}
+__device__ __forceinline__ void ca_hess(const CaHess &h, CaHessLds &l, const double (&hr)[CA_HT], const double *R1,
+                                        const double *R2, bool broken) {
+  const int k = h.k, m = h.m, ld = m + 1, nr = k + 1 + CA_S;
+  double *Hf = h.Hf, *hst = h.hst;
+  const GState &G = h.G;
+  const CaShift &B = h.B;
+  auto &Rr = l.Rr;
+  auto &Hn = l.Hn;
+  auto &rot = l.rot;
+  auto &tl = l.tl;
   const int tid = threadIdx.x;
   if (tid < CA_S * CA_S) {
     const int a = tid / CA_S, b = tid % CA_S;
     double v = 0.0;
 #pragma unroll
-    for (int t = 0; t < CA_S; ++t) v += R2[a * CA_S + t] * R1[t * CA_S + b];
-    Rt[a * CA_S + b] = v;
-  }
-  for (int e = tid; e < 2 * k; e += blockDim.x) rot[e] = G.csn[e];
-  __syncthreads();
-  for (int e = tid; e < nr * (CA_S + 1); e += blockDim.x) {
-    const int r = e % nr, c = e / nr;
-    double v;
-    if (c == 0)
-      v = (r == k) ? 1.0 : 0.0;
-    else if (r <= k)
-      v = C[r * CA_S + (c - 1)];
-    else
-      v = Rt[(r - k - 1) * CA_S + (c - 1)];
-    Rr[c * nr + r] = v;
+    for (int t = 0; t < CA_S; ++t) v += (R2 ? R2[a * CA_S + t] : a == t ? 1.0 : 0.0) * R1[t * CA_S + b];
+    Rr[(b + 1) * nr + k + 1 + a] = v;
   }
   __syncthreads();
-  for (int e = tid; e < (k + 1) * CA_S; e += blockDim.x) {
-    const int r = e % (k + 1), c = e / (k + 1);
-    double v = 0.0;
-    for (int t = (r > 0 ? r - 1 : 0); t < k; ++t) v += Hf[(int64_t)t * ld + r] * Rr[c * nr + t];  // H_old is upper Hessenberg
-    HC[c * (k + 1) + r] = v;
+  {
+    const int r = tid % CA_MAXR, sl = tid / CA_MAXR;
+    if (sl < CA_S) {
+      double p[CA_S];
+#pragma unroll
+      for (int c = 0; c < CA_S; ++c) p[c] = 0.0;
+#pragma unroll
+      for (int j = 0; j < CA_HT; ++j) {
+        const int t = min(sl * CA_HT + j, nr - 1);
+#pragma unroll
+        for (int c = 0; c < CA_S; ++c) p[c] += hr[j] * Rr[c * nr + t];
+      }
+#pragma unroll
+      for (int c = 0; c < CA_S; ++c) l.hp[sl][c][r] = p[c];
+    }
   }
   __syncthreads();
   // Hnew = (Rr Bc - [HC; 0]) T^{-1},  T = Rr[k:k+S, 0:S] upper triangular, Bc the change of basis
@@ -3126,7 +3135,9 @@ __global__ void __launch_bounds__(256) k_ca_hess(int k, int m, const double *__r
     double x[CA_S];
 #pragma unroll
     for (int c = 0; c < CA_S; ++c) {
-      double v = Rr[(c + 1) * nr + r] + B.d[c] * Rr[c * nr + r] - (r <= k ? HC[c * (k + 1) + r] : 0.0);
+      double v = Rr[(c + 1) * nr + r] + B.d[c] * Rr[c * nr + r];
+#pragma unroll
+      for (int sl = 0; sl < CA_S; ++sl) v -= l.hp[sl][c][r];  // zero below row k
       if (c > 0) v -= B.c[c] * Rr[(c - 1) * nr + r];
 #pragma unroll
       for (int t = 0; t < c; ++t) v -= x[t] * Rr[c * nr + (k + t)];
@@ -3146,6 +3157,7 @@ __global__ void __launch_bounds__(256) k_ca_hess(int k, int m, const double *__r
     const int c = tid;
     double *Rc = G.R + (int64_t)(k + c) * ld;
     double a = Hn[c];
+#pragma unroll 5
     for (int t = 0; t < k; ++t) {
       const double b = Hn[(t + 1) * CA_S + c], cs = rot[2 * t], sn = rot[2 * t + 1];
       Rc[t] = cs * a + sn * b;
@@ -3189,11 +3201,121 @@ __global__ void __launch_bounds__(256) k_ca_hess(int k, int m, const double *__r
 #pragma unroll
     for (int i = 0; i <= c + 1; ++i) Rc[i] = v[i];
   }
-  hst[m + 8 + slot] = flag[0];
+  hst[m + 8 + h.slot] = broken ? 1.0 : 0.0;
 }
 
 // One CA-GMRES(m) cycle on the DG operator Ahat (block Jacobi folded in); same contract as
 // gmres_cycle. Returns -1 (and changes nothing in x) if the first block breaks down.
+// W <- W R^{-1} (R upper triangular S x S, row-major), Gram partials of the result if part.
+// The first NXCD blocks of the grid carry no rows (so that the others keep their place on the XCDs):
+// block 0 does the block's Hessenberg columns meanwhile, which need the factor and not W. FAC: the
+// factor is not ready, every block sums the Gram partials (np per entry) and factors for itself;
+// block 0 stores R. All of it is latency: sum, factor and solve, twice, and the columns were seven launches of 2.8,
+// 3.0, 3.8 and once 7.0 us on 27,648 FP64 unknowns with their gaps, now two of 7.0 us (DG-P2 48^2: 15.1 -> 11.8 ms a solve);
+// 786,432 FP32 unknowns: 4.5 + 4.2 + 6.9 + 8.5 us -> 9.8 us after a k_ca_chol of 6.1 (256^2: 150.9 -> 140.7 ms).
+struct CaFactor {
+  const double *gpart;
+  int np;
+  const double *Rinv;  // !FAC
+  double *R;           // FAC: where block 0 leaves the factor
+  double *flag;
+};
+template <typename T, bool FAC>
+__global__ void __launch_bounds__(NTHR) k_btrsm_gram(int64_t n, T *__restrict__ W, int64_t ldv, CaFactor F, CaHess H,
+                                                     double *__restrict__ part) {
+  constexpr int VW = Vec<T>::w;
+  __shared__ double ri[CA_S * CA_S], rl[CA_S * CA_S], gs[CA_NG];
+  __shared__ int ok;
+  __shared__ double sh[NTHR / 64][CA_NG + 1];
+  __shared__ CaHessLds hl;
+  const int nb = gridDim.x - NXCD;  // blocks with rows, a multiple of NXCD
+  const int rb = (int)blockIdx.x - NXCD;
+  if (rb < 0 && rb != -NXCD) return;
+  const int lb = (rb % NXCD) * (nb / NXCD) + rb / NXCD;  // xcd_block() of the others
+  const int64_t nvec = n / VW;
+  const int64_t chunk = (nvec + nb - 1) / nb;
+  const int64_t i0 = lb * chunk, i1 = min(nvec, i0 + chunk);
+  int64_t i = i0 + threadIdx.x;
+  T wv[CA_S][VW];  // the first rows, under way while the factor is made
+  if (rb >= 0 && i < i1)
+#pragma unroll
+    for (int t = 0; t < CA_S; ++t) vload(W + (int64_t)t * ldv + i * VW, wv[t]);
+  double hr[CA_HT];
+  if (rb < 0 && H.on) ca_hess_load(H, hl, hr);
+  if constexpr (FAC) {
+    ca_factor_block<NTHR / 64>(F.gpart, F.np, gs, rl, ri, &ok);
+  } else {
+    if (rb >= 0 && (int)threadIdx.x < CA_S * CA_S) ri[threadIdx.x] = F.Rinv[threadIdx.x];
+    __syncthreads();
+  }
+  if (rb < 0) {
+    bool broken = false;
+    if constexpr (FAC) {
+      if ((int)threadIdx.x < CA_S * CA_S) F.R[threadIdx.x] = rl[threadIdx.x];
+      if (threadIdx.x == 0 && !ok) F.flag[0] = 1.0;
+      broken = !ok;
+    }
+    if (!H.on) return;
+    const double *R1 = H.R1, *R2 = H.R2;
+    if constexpr (FAC) (R2 ? R2 : R1) = rl;
+    ca_hess(H, hl, hr, R1, R2, broken || F.flag[0] != 0.0);
+    return;
+  }
+  double gacc[CA_NG];
+#pragma unroll
+  for (int g = 0; g < CA_NG; ++g) gacc[g] = 0.0;
+  for (; i < i1; i += blockDim.x) {
+    if (i != i0 + threadIdx.x)
+#pragma unroll
+      for (int t = 0; t < CA_S; ++t) vload(W + (int64_t)t * ldv + i * VW, wv[t]);
+    T ov[CA_S][VW];
+#pragma unroll
+    for (int l = 0; l < VW; ++l)
+#pragma unroll
+      for (int t = 0; t < CA_S; ++t) {
+        double sum = 0.0;
+#pragma unroll
+        for (int a = 0; a <= t; ++a) sum += (double)wv[a][l] * ri[a * CA_S + t];
+        ov[t][l] = (T)sum;
+      }
+#pragma unroll
+    for (int t = 0; t < CA_S; ++t) vstore(W + (int64_t)t * ldv + i * VW, ov[t]);
+    if (part) {
+#pragma unroll
+      for (int l = 0; l < VW; ++l) {
+        int g = 0;
+#pragma unroll
+        for (int a = 0; a < CA_S; ++a)
+#pragma unroll
+          for (int b = a; b < CA_S; ++b, ++g) gacc[g] += (double)ov[a][l] * (double)ov[b][l];
+      }
+    }
+  }
+  if (lb == nb - 1)
+    for (int64_t i = nvec * VW + threadIdx.x; i < n; i += blockDim.x) {
+      double w[CA_S];
+      T o[CA_S];
+      for (int t = 0; t < CA_S; ++t) w[t] = (double)W[(int64_t)t * ldv + i];
+      for (int t = 0; t < CA_S; ++t) {
+        double sum = 0.0;
+        for (int a = 0; a <= t; ++a) sum += w[a] * ri[a * CA_S + t];
+        o[t] = (T)sum;
+        W[(int64_t)t * ldv + i] = o[t];
+      }
+      if (part) {
+        int g = 0;
+        for (int a = 0; a < CA_S; ++a)
+          for (int b = a; b < CA_S; ++b, ++g) gacc[g] += (double)o[a] * (double)o[b];
+      }
+    }
+  if (!part) return;
+  double v[CA_NG + 1];  // (padded to an even number, which sums in fewer exchanges)
+#pragma unroll
+  for (int g = 0; g < CA_NG; ++g) v[g] = gacc[g];
+  v[CA_NG] = 0.0;
+  block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, nb);
+}
+
 template <typename T>
 static int ca_gmres_cycle(Matrix *A, Precond *P, const double *r0, double beta, double *x, int m, double stop_abs,
                           int maxit, Work &w, bool &breakdown, CaShift &shift, bool &newton) {
@@ -3220,9 +3342,18 @@ static int ca_gmres_cycle(Matrix *A, Precond *P, const double *r0, double beta, 
   const int grid = stream_grid((n + VW - 1) / VW);
   // the block dot reduces CA_KQ x CA_S sums per block: fewer, longer blocks amortise that
   // the block dot runs on a quarter of the streaming grid per y-tile (measured 88 us against
-  // 91 us at half and 117 us at the full grid, DG-P2 512^2 FP32): fewer, longer row streams
-  const int dgrid = std::max(NXCD, grid / 4 / NXCD * NXCD);
-  ensure_part(w, (size_t)(m + 1) * CA_S * grid + 64);
+  // 91 us at half and 117 us at the full grid, DG-P2 512^2 FP32): fewer, longer row streams; a small system
+  // keeps 56 blocks, below which a thread's rows become a chain (DG-P2 48^2 FP64: 5.9 us, 8.6 with 8 blocks)
+  const int dgrid = std::min(grid, std::max(56, grid / 4 / NXCD * NXCD));
+  // (the partials of the coefficients and of the two Gram matrices of a block lie side by side: a kernel
+  // may sum one while it writes the next)
+  const size_t npc = (size_t)(m + 1) * CA_S * dgrid;
+  ensure_part(w, std::max((size_t)(m + 1) * CA_S * grid + 64, npc + 2 * (size_t)CA_NG * grid));
+  double *gp1 = w.part.p + npc, *gp2 = gp1 + (size_t)CA_NG * grid;
+  // every block of the triangular solve factors for itself up to CA_FAC_BLOCKS partials an entry: DG-P2 96^2
+  // FP64 (216 partials) 21.0 ms a solve against 21.9 with a launch for it, 200^2 FP32 (472) 76.4 against 77.2,
+  // 256^2 FP32 (768) 140.7 against 141.4; beyond, each block would read more for it than of its rows
+  const bool fac = grid <= CA_FAC_BLOCKS;
   k_scale_copy<double, T><<<nblk(n), NTHR, 0, st>>>(n, r0, 1.0 / beta, Q);
   // g = e_0 (relative to beta), flag = 0, one = 1
   k_gmres_init<<<1, 64, 0, st>>>(m, 1.0, g, flag, 0.0, nullptr);
@@ -3305,25 +3436,26 @@ static int ca_gmres_cycle(Matrix *A, Precond *P, const double *r0, double beta, 
     reduce_to(w.part.p, dgrid, nq * CA_S, Cm, st);
     {
       KTimer tm(ctx, c_upd, (double)(nq + 2 * CA_S) * n * sizeof(T));
-      k_bupdate_gram<T><<<grid, NTHR, 0, st>>>(n, Q, ldv, nq, W, Cm, w.part.p);
+      k_bupdate_gram<T><<<grid, NTHR, 0, st>>>(n, Q, ldv, nq, W, Cm, gp1);
     }
-    double *gp = Cm + (size_t)(m + 1) * CA_S - CA_NG;  // packed Gram (the last rows of Cm are unused: nq <= m+1-S)
-    reduce_to(w.part.p, grid, CA_NG, gp, st);
     {
       // CholQR, and a second pass (CholQR2) for FP64 bases only: the shifted blocks have Gram
       // condition ~1e4, so one pass leaves FP32 vectors orthogonal to ~1e-6, below their precision
       KTimer tm(ctx, c_qr, (sizeof(T) == 8 ? 4.0 : 2.0) * CA_S * n * sizeof(T));
-      k_ca_chol<<<1, 64, 0, st>>>(gp, R1, R1i, flag, sizeof(T) == 8 ? nullptr : R2);
-      if (sizeof(T) == 8) {
-        k_btrsm_gram<T><<<grid, NTHR, 0, st>>>(n, W, ldv, R1i, w.part.p);
-        reduce_to(w.part.p, grid, CA_NG, gp, st);
-        k_ca_chol<<<1, 64, 0, st>>>(gp, R2, R2i, flag, nullptr);
-        k_btrsm_gram<T><<<grid, NTHR, 0, st>>>(n, W, ldv, R2i, nullptr);
-      } else {
-        k_btrsm_gram<T><<<grid, NTHR, 0, st>>>(n, W, ldv, R1i, nullptr);
+      constexpr int NPASS = sizeof(T) == 8 ? 2 : 1;
+      for (int ps = 0; ps < NPASS; ++ps) {
+        const bool last = ps + 1 == NPASS;
+        double *R = ps == 0 ? R1 : R2, *Ri = ps == 0 ? R1i : R2i;
+        const double *gp = ps == 0 ? gp1 : gp2;
+        if (!fac) k_ca_chol<<<1, 1024, 0, st>>>(gp, grid, R, Ri, flag);
+        const CaFactor F{gp, grid, Ri, R, flag};
+        const CaHess H{last ? 1 : 0, k, m, bidx & 1, Cm, R1, NPASS == 2 ? R2 : nullptr, Hf, G, shift, hres_d};
+        if (fac)
+          k_btrsm_gram<T, true><<<grid + NXCD, NTHR, 0, st>>>(n, W, ldv, F, H, last ? nullptr : gp2);
+        else
+          k_btrsm_gram<T, false><<<grid + NXCD, NTHR, 0, st>>>(n, W, ldv, F, H, last ? nullptr : gp2);
       }
     }
-    k_ca_hess<<<1, 256, 0, st>>>(k, m, Cm, R1, R2, Hf, G, shift, flag, hres_d, bidx & 1);
     const int ev = bidx & 1;
     OCMP_HIP(hipEventRecord(work_event(w, ev), st));
     inflight.push_back({k, ev});
