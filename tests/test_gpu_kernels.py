@@ -243,3 +243,136 @@ def test_unet_tiles(gpu_ctx, N):
         for size in (ci * co * 27, co):
             assert rel(g[o:o + size], gt[o:o + size]) < 1e-5, name
             o += size
+
+
+# ------------------------------------------------------------------------------------------ MLP tiles
+
+
+# 64 rows a wave from 131,072 rows: the first of them with and without a rest, and one past a whole block
+@pytest.mark.parametrize('n', [127, 129, 130944, 130945, 131072, 131073 + 63, 262145])
+def test_mlp_rows(gpu_ctx, n):
+    """Forward and guess against the oracle; 2e-3 bounds the bf16 roundings that an FP32 sum puts one unit
+    apart (as in the tests of the network)."""
+    import torch
+    from oracle import mlp as om
+    from opencmp_amd.learned import MLPGuess
+    p = om.init_params(3).astype(np.float32)
+    net = MLPGuess(gpu_ctx, params=p, max_batch=128)
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 4)).astype(np.float32)
+    y = net.forward(torch.from_numpy(X).cuda()).cpu().numpy().astype(np.float64)
+    yo = om.forward(p, X, bf16=True)
+    assert rel(y, yo) <= 2e-3
+    tail = slice(n - min(n, 70), n)     # the last rows on their own: a wrong rest hides in the norm
+    assert rel(y[tail], yo[tail]) <= 1e-2
+    u = [rng.standard_normal(n) for _ in range(4)]
+    off, sc, U = [0, n // 3, n], [0.5, 2.0], [1.0, 1.5]
+    net.set_scales(off, sc, U)
+    g = net.guess([torch.from_numpy(v).cuda() for v in u]).cpu().numpy()
+    go = om.guess(p, u, off, sc, U, bf16=True)
+    assert rel(g - u[0], go - u[0]) <= 2e-3
+
+
+@pytest.mark.parametrize('B', [1, 63, 65, 257, 16385])
+def test_mlp_gradient_rows(gpu_ctx, B):
+    """Chunks of 64 rows, blocks of 256, of 64 rows or more for the small sums; 2e-2 as above for gradients."""
+    import torch
+    from oracle import mlp as om
+    from opencmp_amd.learned import MLPGuess
+    p = om.init_params(5).astype(np.float32)
+    net = MLPGuess(gpu_ctx, params=p, max_batch=B)
+    rng = np.random.default_rng(B)
+    X = rng.standard_normal((B, 4)).astype(np.float32)
+    T = rng.standard_normal(B).astype(np.float32)
+    g, loss = net.grad(torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda())
+    lo, go = om.loss_and_grad(p, X, T, bf16=True)
+    g = g.cpu().numpy()
+    assert rel(g, go) <= 2e-2 and abs(loss - lo) <= 1e-3 * lo
+
+
+# ------------------------------------------------------------------------------------------ solvers' forms
+
+
+def _apply(a, x):
+    import torch
+    y = torch.empty_like(x)
+    a.mult(x, y)
+    return y
+
+
+def _poisson(C, ctx, n, kappa):
+    fes = C.FESpace(C.Mesh(unit_square(n), ctx), [C.H1(2, 'left|top')])
+    a = C.BilinearForm(fes, [C.Vol('gradgrad', 0, 0, coef=kappa)])
+    f = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, POLY[2]))])
+    return fes, a, f
+
+
+# scalars summed by every block (up to 512 row blocks), by one block in its own launch beyond 2048
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('n', [2, 40, 240, 520])
+def test_cg_forms(gpu_ctx, n, precision):
+    """The solution solves the system: residual of the returned vector, by the operator's own product."""
+    import torch
+    C = core()
+    fes, a, f = _poisson(C, gpu_ctx, n, 1.3)
+    a.Assemble()
+    f.Assemble()
+    pre = C.Preconditioner(a, 'local', precision=precision)
+    pre.Update()
+    u = C.GridFunction(fes)
+    tol = 1e-9
+    st = C.solve(a, f.vec, u.vec, pre, 'CG', tol=tol, precision=precision,
+                 inner_tol=1e-4 if precision == 'mixed' else 0.0)
+    assert st.converged
+    free = torch.from_numpy(fes.FreeDofs()).to(u.vec.device)
+    y = _apply(a, u.vec)
+    r = torch.where(free, f.vec - y, torch.zeros_like(y))
+    b = torch.where(free, f.vec, torch.zeros_like(y))
+    # the stopping rule bounds the recurred residual; the true one is off by its rounding, some units of
+    # 1.1e-16 |A| |x| with |A| <= 40 (rows of the P2 stiffness matrix, kappa = 1.3)
+    assert float(r.norm()) <= 1.01 * tol * float(b.norm()) + 1e-15 * 40 * float(u.vec.norm())
+
+
+# the s-step factor made by every block (up to 1024 Gram partials an entry) and in its own launch
+@pytest.mark.parametrize('n,precision', [(2, 'fp64'), (17, 'fp64'), (17, 'mixed'), (216, 'fp64')])
+def test_s_step_blocks(gpu_ctx, n, precision):
+    import torch
+    C = core()
+    hm = unit_square(n)
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.L2(2)], dgjumps=True)
+    a = C.BilinearForm(fes, [C.Vol('mass', 0, 0, coef=400.0), C.Vol('gradgrad', 0, 0, coef=1e-3),
+                             C.DGFacet(0, eps=1e-3, alpha=40.0, dirichlet=hm.marker_mask(hm.bnd_names))])
+    f = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, POLY[2]))])
+    a.Assemble()
+    f.Assemble()
+    pre = C.Preconditioner(a, 'local', precision=precision)
+    pre.Update()
+    u = C.GridFunction(fes)
+    st = C.solve(a, f.vec, u.vec, pre, 'GMRes', tol=1e-9, restart=50, precision=precision,
+                 inner_tol=1e-4 if precision == 'mixed' else 0.0, s_step=5)
+    assert st.converged and not st.fallback
+    r = f.vec - _apply(a, u.vec)
+    assert float(r.norm()) <= 1.01e-9 * float(f.vec.norm())
+
+
+def test_kept_plans_follow_the_form(gpu_ctx):
+    """A form assembled again takes the coefficients, sources and field values of the moment, also after
+    another form of the same space was assembled in between."""
+    import torch
+    C = core()
+    fes, a, f = _poisson(C, gpu_ctx, 9, 1.0)
+    a2 = C.BilinearForm(fes, [C.Vol('gradgrad', 0, 0, coef=2.5), C.Vol('mass', 0, 0, coef=1.0)])
+    f2 = C.LinearForm(fes, [C.Source(0, (L.FN_POLY2, [2.0 * c for c in POLY[2]]))])
+    x = torch.linspace(-1, 1, fes.ndof, dtype=torch.float64, device='cuda')
+    a.Assemble()
+    y1 = _apply(a, x).clone()
+    a2.Assemble()
+    a.Assemble()
+    assert torch.equal(_apply(a, x), y1)
+    f.Assemble()
+    b1 = f.vec.clone()
+    f2.Assemble()
+    f.Assemble()
+    assert torch.equal(f.vec, b1)
+    # twice the source is twice the vector, to the rounding of its sums
+    assert float((f2.vec - 2 * b1).abs().max()) <= 1e-15 * float(b1.abs().max()) * 8
