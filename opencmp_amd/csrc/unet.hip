@@ -198,8 +198,8 @@ __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
 // as the fourth such group, the bias), its wavefronts quarters of the chunk: each lane loads four
 // consecutive voxels of channel a = l % 16 once and the shifted voxels of channel b = l % 16 for
 // every tap, and v_mfma_f32_16x16x4 contracts voxel by voxel. Fixed partitions and order of sums.
-// 33^3 grid: 95 us and 20 for the sums, against 426 us in 32 launches (one per layer, operand and
-// stage, on the vector units).
+// 33^3 grid: 62 us (95 with a branch around each load) and 20 for the sums, against 426 us in 32 launches (one
+// per layer, operand and stage, on the vector units).
 struct WGrad {
   const void *P, *Q, *G;
   int p_bf16, na, np, q_bf16, nb, nq, stride;
@@ -254,34 +254,52 @@ __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__
   f32x4 acc[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int64_t zb = z0 + wv * 16; zb < z1; zb += 64) {
-    const int64_t zl = zb + 4 * lk;
-    const int64_t zc = min(zl, zp - 1);
-    int zx = (int)(zc % g.np), zt = (int)(zc / g.np), zy = zt % g.np, zz = zt / g.np;
+  // the 40 loads of four voxels go out together: what lies outside reads the channel's first value and counts 0
+  auto sweep = [&](auto *P, auto *Q) {
+    for (int64_t zb = z0 + wv * 16; zb < z1; zb += 64) {
+      const int64_t zl = zb + 4 * lk;
+      const int zc = (int)min(zl, zp - 1);
+      int zx = zc % g.np, zt = zc / g.np, zy = zt % g.np, zz = zt / g.np;
+      float pv[4], qv[4][9];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool in = zl + r < z1;
-      const float pv = in && a < g.na ? ld_any(g.P, g.p_bf16, pa + zl + r) : 0.f;
-      const int sx = g.stride * zx - 1, sy = g.stride * zy - 1, sz = g.stride * zz + dz - 1;
-      const bool vz = in && b < g.nb && sz >= 0 && sz < g.nq;
-      const int64_t row = qb + ((int64_t)sz * g.nq + sy) * g.nq + sx;
-      float qv[9];
+      for (int r = 0; r < 4; ++r) {
+        const bool in = zl + r < z1;
+        const float pr = ld_f(P, pa + (in ? zl + r : 0));
+        pv[r] = (in & (a < g.na)) ? pr : 0.f;
+        const int sx = g.stride * zx - 1, sy = g.stride * zy - 1, sz = g.stride * zz + dz - 1;
+        const bool vz = in & (b < g.nb) & ((unsigned)sz < (unsigned)g.nq);
+        const int row = (sz * g.nq + sy) * g.nq + sx;  // a channel has at most 513^3 voxels
 #pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        const int dy = k / 3, dx = k % 3;
-        const bool ok = vz && sy + dy >= 0 && sy + dy < g.nq && sx + dx >= 0 && sx + dx < g.nq;
-        qv[k] = ok ? ld_any(g.Q, g.q_bf16, row + (int64_t)dy * g.nq + dx) : 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < 9; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(pv, qv[k], acc[k], 0, 0, 0);
-      if (++zx == g.np) {
-        zx = 0;
-        if (++zy == g.np) {
-          zy = 0;
-          ++zz;
+        for (int k = 0; k < 9; ++k) {
+          const int dy = k / 3, dx = k % 3;
+          const bool ok = vz & ((unsigned)(sy + dy) < (unsigned)g.nq) & ((unsigned)(sx + dx) < (unsigned)g.nq);
+          const float q = ld_f(Q, qb + (ok ? row + dy * g.nq + dx : 0));
+          qv[r][k] = ok ? q : 0.f;
+        }
+        if (++zx == g.np) {
+          zx = 0;
+          if (++zy == g.np) {
+            zy = 0;
+            ++zz;
+          }
         }
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < 9; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[r], qv[r][k], acc[k], 0, 0, 0);
     }
+  };
+  if (g.p_bf16) {
+    if (g.q_bf16)
+      sweep((const u16 *)g.P, (const u16 *)g.Q);
+    else
+      sweep((const u16 *)g.P, (const float *)g.Q);
+  } else {
+    if (g.q_bf16)
+      sweep((const float *)g.P, (const u16 *)g.Q);
+    else
+      sweep((const float *)g.P, (const float *)g.Q);
   }
 #pragma unroll
   for (int k = 0; k < 9; ++k)
