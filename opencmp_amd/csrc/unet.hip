@@ -122,8 +122,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // holds weight (channel l % 16, input l / 16) and input (input l / 16, voxel l % 16): both loads
 // are runs of 16, and it receives channels 4 (l / 16) + r, r = 0..3, of voxel l % 16. What bounds the
 // coarse levels is one wavefront's chain of dependent loads (9^3 voxels are 46 tiles): hence the split
-// of the taps. 33^3 grid, all 23 products of two forwards and a gradient: 261 us (one thread per
-// voxel and 8 channels, weights staged in LDS by every workgroup: 1745 us).
+// of the taps, and all of a wavefront's loads before its first product. 33^3 grid, all 23 products of two
+// forwards and a gradient: 192 us (tap after tap 261; one thread per voxel and 8 channels, weights staged in
+// LDS by every workgroup: 1745 us).
 template <int CIN, typename TI>
 __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
   __shared__ float sh[4][256];
@@ -137,10 +138,16 @@ __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
     const int64_t zr = z < zout ? z : zout - 1;
     const int zx = (int)(zr % c.nout), zq = (int)(zr / c.nout), zy = zq % c.nout, zz = zq / c.nout;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k = wv; k < 27; k += 4) {
+    // a wave's seven taps: all loads first, then the matrix instructions
+    constexpr int NTAP = 7;
+    float x[NTAP][CIN / 4], w[NTAP][CIN / 4];
+    bool ok[NTAP], any[NTAP];
+#pragma unroll
+    for (int j = 0; j < NTAP; ++j) {
+      const int k = wv + 4 * j;
       const int dz = k / 9, dy = (k / 3) % 3, dx = k % 3;
       int sx, sy, sz;
-      bool ok = z < zout;
+      bool in_ = z < zout && k < 27;
       if (!c.transposed) {
         sx = c.stride * zx + dx - 1;
         sy = c.stride * zy + dy - 1;
@@ -148,7 +155,7 @@ __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
       } else {
         const int tx = zx - dx + 1, ty = zy - dy + 1, tz = zz - dz + 1;
         if (c.stride == 2) {
-          ok = ok && !((tx | ty | tz) & 1);
+          in_ = in_ && !((tx | ty | tz) & 1);
           sx = tx >> 1;
           sy = ty >> 1;
           sz = tz >> 1;
@@ -158,19 +165,22 @@ __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
           sz = tz;
         }
       }
-      ok = ok && sx >= 0 && sy >= 0 && sz >= 0 && sx < c.nin && sy < c.nin && sz < c.nin;
-      if (!__any(ok)) continue;  // whole wavefront: the matrix instructions below run with all lanes
-      const int64_t src = ok ? ((int64_t)sz * c.nin + sy) * c.nin + sx : 0;
-      float x[CIN / 4], w[CIN / 4];
+      ok[j] = in_ && sx >= 0 && sy >= 0 && sz >= 0 && sx < c.nin && sy < c.nin && sz < c.nin;
+      any[j] = __any(ok[j]);  // whole wavefront: the matrix instructions below run with all lanes
+      const int64_t src = ok[j] ? ((int64_t)sz * c.nin + sy) * c.nin + sx : 0;
+      if (any[j])
 #pragma unroll
-      for (int i = 0; i < CIN / 4; ++i) {
-        x[i] = ld_f(in, (int64_t)(4 * i) * zin + src);
-        w[i] = W[(int64_t)(k * CIN + 4 * i) * c.cop];
-      }
-#pragma unroll
-      for (int i = 0; i < CIN / 4; ++i)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], ok ? x[i] : 0.f, acc, 0, 0, 0);
+        for (int i = 0; i < CIN / 4; ++i) {
+          x[j][i] = ld_f(in, (int64_t)(4 * i) * zin + src);
+          w[j][i] = W[(int64_t)(k * CIN + 4 * i) * c.cop];
+        }
     }
+#pragma unroll
+    for (int j = 0; j < NTAP; ++j)
+      if (any[j])
+#pragma unroll
+        for (int i = 0; i < CIN / 4; ++i)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][i], ok[j] ? x[j][i] : 0.f, acc, 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) sh[wv][r * 64 + lane] = acc[r];
   }
