@@ -1796,6 +1796,13 @@ static DBuf<double> *cached_table(Space &s, const std::string &key, const TableB
   return buf;
 }
 
+// A key names everything that a table's contents and layout depend on, by value: of a field that is the
+// element of its block (never its space's address, which a later space of another order may have)
+static std::string field_key(const ocmp_field &f) {
+  const Block &b = f.space->s.blocks[f.block];
+  return "|f" + std::to_string(b.kind) + "," + std::to_string(b.order);
+}
+
 static std::string term_key(const std::vector<ocmp_term> &terms, const std::vector<ocmp_field> &fields) {
   std::string k = "B";
   for (auto &t : terms) {
@@ -1803,8 +1810,14 @@ static std::string term_key(const std::vector<ocmp_term> &terms, const std::vect
     k += "|" + std::to_string(t.kind) + "," + std::to_string(t.trial) + "," + std::to_string(t.test) + "," +
          std::to_string(quad);
   }
-  for (auto &f : fields) k += "|f" + std::to_string((uintptr_t)f.space) + "," + std::to_string(f.block);
+  for (auto &f : fields) k += field_key(f);
   return k;
+}
+
+// the field whose basis a volume term's gather tables contain: its wind or its weight (NULL: neither)
+static const ocmp_field *table_field(const ocmp_term &t, const std::vector<ocmp_field> &fields) {
+  if (t.kind == OCMP_BFI_CONV && t.wind_field >= 0) return &fields[t.wind_field];
+  return t.weight_mode != OCMP_WEIGHT_NONE ? &fields[t.weight_field] : nullptr;
 }
 
 // phi of a (kind, order) block at the facet rules of all local facets (facet k opposite vertex k):
@@ -1926,12 +1939,10 @@ static std::vector<double> gather_tables(const Space &s, const ocmp_term &t, con
                                          int &nf) {
   const int d = s.mesh->dim;
   const Block &bt = s.blocks[t.test], &bj = s.blocks[t.trial];
-  const bool wind_field = t.kind == OCMP_BFI_CONV && t.wind_field >= 0;
-  const bool weighted = t.weight_mode != OCMP_WEIGHT_NONE;
+  const ocmp_field *f = table_field(t, fields);
   int fo = 0, nw = 1, fkind = 0;
-  if (wind_field || weighted) {
-    const ocmp_field &f = fields[wind_field ? t.wind_field : t.weight_field];
-    const Block &fb = f.space->s.blocks[f.block];
+  if (f) {
+    const Block &fb = f->space->s.blocks[f->block];
     fo = fb.order;
     nw = fb.nloc;
     fkind = fb.kind;
@@ -1953,7 +1964,7 @@ static std::vector<double> gather_tables(const Space &s, const ocmp_term &t, con
     const double *lam = &rule.lam[q * (d + 1)];
     eval_basis(bt.kind, d, bt.order, lam, pt.data(), gt.data());
     eval_basis(bj.kind, d, bj.order, lam, pj.data(), gj.data());
-    if (wind_field || weighted)
+    if (f)
       eval_basis(fkind, d, fo, lam, pw.data(), gw.data());
     else
       pw[0] = 1.0;
@@ -2150,9 +2161,12 @@ static bool gather_plan(Matrix *M, const std::vector<ocmp_term> &vol, const std:
   }
   if (maxpf > 64) return false;
   KF.NF = NF;
-  // (which terms share a factor set decides the tables' layout)
-  std::string key = "G" + term_key(vol, fields);
-  for (int si : term_set) key += "," + std::to_string(si);
+  // which field a term takes decides its tables, and which terms share a factor set their layout
+  std::string key = "G" + term_key(vol, {});
+  for (size_t ti = 0; ti < vol.size(); ++ti) {
+    const ocmp_field *f = table_field(vol[ti], fields);
+    key += (f ? field_key(*f) : "|-") + "," + std::to_string(term_set[ti]);
+  }
   DBuf<double> *tab = cached_table(s, key, tb, st);
   KG.NL = s.nloc;
   KG.NF = NF;
@@ -2588,7 +2602,7 @@ static LinPlan linear_plan(Space &s, const std::vector<ocmp_lterm> &terms, const
   std::string key = "L" + std::to_string(qdeg);
   for (auto &t : terms) key += "|" + std::to_string(t.kind) + "," + std::to_string(t.test) + "," +
                                std::to_string(t.fn) + "," + std::to_string(t.fn == OCMP_FN_FIELD ? t.field : -1);
-  for (auto &f : fields) key += "|f" + std::to_string((uintptr_t)f.space) + "," + std::to_string(f.block);
+  for (auto &f : fields) key += field_key(f);
   DBuf<double> *tab = cached_table(s, key, tb, st);
   A.tab = tab->p;
   for (auto &t : terms) P.has_src |= t.kind == OCMP_LFI_SOURCE;

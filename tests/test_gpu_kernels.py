@@ -198,6 +198,75 @@ def test_gather_units(gpu_ctx, make, order):
     assert rel(gpu([G(1.0)] * 31 + [M(1.0), X(1.0)]), ref(31.0, 1.0, 1.0)) < 1e-13
 
 
+def _field_case(C, ctx, gm, hm, t, order, seed, ncomp=1):
+    """A grid function of random values on a space of its own, and the oracle's evaluation of it."""
+    import torch
+    fes = C.FESpace(gm, [C.H1(order, ncomp=ncomp)])
+    v = np.random.default_rng(seed).standard_normal(fes.ndof)
+    gf = C.GridFunction(fes, torch.tensor(v, device=ctx.torch_device))
+    return gf, fem.GridFunctionEval(fem.Space(t, 'H1', order, ncomp=ncomp), v)
+
+
+def _assert_volume(C, fes, cs, terms, ref):
+    a = C.BilinearForm(fes, terms)
+    a.Assemble()
+    A = fem.Assembler(cs)
+    fem.assemble_volume(A, ref, qdeg=8)     # exact: P2 test and trial, a P3 weight
+    r = A.matrix().data
+    assert rel(a.values(), r) < 1e-13
+
+
+def test_tables_of_the_weighting_field(gpu_ctx):
+    """Forms of one space with the same list of fields, whose last term is weighted by the P1 field in
+    one and by the P2 or P3 field in the others: each has tables of its own."""
+    C = core()
+    hm = unit_square(4)
+    gm, t = C.Mesh(hm, gpu_ctx), fem.Topology(hm)
+    fes, cs = C.FESpace(gm, [C.H1(2)]), fem.Compound([fem.Space(t, 'H1', 2)])
+    f = [_field_case(C, gpu_ctx, gm, hm, t, p, p) for p in (1, 2, 3)]
+    for k in (0, 1, 2, 0):
+        terms = [C.Vol('mass', 0, 0, weight_gf=(gf, 0, L.WEIGHT_FIELD)) for gf, _ in f] + \
+                [C.Vol('gradgrad', 0, 0, coef=2.0, weight_gf=(f[k][0], 0, L.WEIGHT_FIELD))]
+        ref = [dict(kind='mass', trial=0, test=0, coef=('field', e, 1, 1.0)) for _, e in f] + \
+              [dict(kind='grad_grad', trial=0, test=0, coef=('field', f[k][1], 1, 2.0))]
+        _assert_volume(C, fes, cs, terms, ref)
+
+
+@pytest.mark.parametrize('path', ['row gather', 'element scatter', 'load vector'])
+def test_tables_of_a_later_field_space(gpu_ctx, path):
+    """Spaces of fields that come and go, each of another order than the one before it and mostly at its
+    address: no table of an earlier one is taken."""
+    import gc
+    C = core()
+    hm = unit_square(4)
+    gm, t = C.Mesh(hm, gpu_ctx), fem.Topology(hm)
+    fes, cs = C.FESpace(gm, [C.H1(2)]), fem.Compound([fem.Space(t, 'H1', 2)])
+    for order in (1, 3, 2, 1):
+        gf, e = _field_case(C, gpu_ctx, gm, hm, t, order, order)
+        if path == 'row gather':
+            _assert_volume(C, fes, cs, [C.Vol('gradgrad', 0, 0, coef=2.0, weight_gf=(gf, 0, L.WEIGHT_FIELD))],
+                           [dict(kind='grad_grad', trial=0, test=0, coef=('field', e, 1, 2.0))])
+        elif path == 'element scatter':
+            # a wind and a weight in one term; the quadrature follows the weight's order
+            w, ew = _field_case(C, gpu_ctx, gm, hm, t, 1, 7, ncomp=2)
+            _assert_volume(C, fes, cs, [C.Vol('conv', 0, 0, wind_gf=(w, w.space.comp_blocks[0]),
+                                              weight_gf=(gf, 0, L.WEIGHT_FIELD))],
+                           [dict(kind='conv', trial=0, test=0, coef=('field', e, 1, 1.0), wind=ew)])
+            del w
+        else:
+            b = C.LinearForm(fes, [C.Source(0, field_gf=(gf, 0), weight_gf=(gf, 0, L.WEIGHT_FIELD))])
+            b.Assemble()
+            lam, w = fem.simplex_rule(2, 8)
+            phi, _ = fem.ref_basis('H1', 2, 2, lam)
+            c = e.at(lam)[0][..., 0] ** 2 * (w[None, :] * t.absdet[:, None])
+            ref = np.zeros(cs.ndof)
+            np.add.at(ref, cs.spaces[0].edofs1, np.einsum('eq,qi->ei', c, phi))
+            assert rel(b.vec.cpu().numpy(), ref) < 1e-13
+            del b
+        del gf
+        gc.collect()
+
+
 # ------------------------------------------------------------------------------------------ U-net
 
 
