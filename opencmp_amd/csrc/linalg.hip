@@ -397,7 +397,9 @@ __device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, 
     }
     __syncthreads();
     if (active) {
-      if (p0 < d || p0 + PER > end) {  // a run with entries of a neighbouring block
+      // a run with entries of a neighbouring block: they count as 0 times 0, whatever x is
+      const bool edge = p0 < d || p0 + PER > end;
+      if (edge) {
 #pragma unroll
         for (int k = 0; k < PER; ++k)
           if (p0 + k < d || p0 + k >= end) {
@@ -408,6 +410,11 @@ __device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, 
       XT xv[PER];
 #pragma unroll
       for (int k = 0; k < PER; ++k) xv[k] = S.xs[R.li[k]];
+      if (edge) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+          if (p0 + k < d || p0 + k >= end) xv[k] = (XT)0;
+      }
       const unsigned m = S.ends[tid];
       int row = S.row[tid];
       XT s = (XT)0;

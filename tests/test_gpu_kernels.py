@@ -136,6 +136,28 @@ def test_spmv_row_blocks(gpu_ctx, name, make, order):
         assert r.converged and r.rel_residual <= 1e-10
 
 
+def test_spmv_infinite_x(gpu_ctx):
+    """An infinite entry of x reaches the rows that have its column, and no other: every column in turn
+    (rows in blocks, so the first and last thread of a block see its neighbours' nonzeros)."""
+    import torch
+    C = core()
+    fes = C.FESpace(C.Mesh(unit_square(13), gpu_ctx), [C.H1(3)])
+    a = C.BilinearForm(fes, [C.Vol('gradgrad', 0, 0), C.Vol('mass', 0, 0)])
+    a.Assemble()
+    rp, col = a.pattern()
+    has = np.zeros((fes.ndof, fes.ndof), bool)
+    has[np.repeat(np.arange(fes.ndof), np.diff(rp)), col] = True
+    finite = torch.empty((fes.ndof, fes.ndof), dtype=torch.bool, device='cuda')
+    x = torch.ones(fes.ndof, dtype=torch.float64, device='cuda')
+    y = gpu_ctx.zeros(fes.ndof)
+    for j in range(fes.ndof):
+        x[j] = float('inf')
+        a.mult(x, y)
+        finite[:, j] = torch.isfinite(y)
+        x[j] = 1.0
+    assert np.array_equal(finite.cpu().numpy(), ~has)
+
+
 @pytest.mark.parametrize('precision', ['fp64', 'mixed'])
 def test_spmv_rows_without_nonzeros(gpu_ctx, precision):
     """FGMRES multiplies by the operator without untouched block pairs: with terms on one of two
