@@ -294,7 +294,7 @@ static RbCsr<T> rb_csr(const Matrix *A, const RowBlocks &rb, const T *val) {
 // LDS of one row block
 template <typename XT, int NNZB, int NT>
 struct RbLds {
-  XT xs[RB_XCAP];            // x at the distinct columns
+  XT xs[RB_XCAP + 1];        // x at the distinct columns, and a zero
   XT fin[RB_ROWS];           // per row: the sum of its last run's part
   XT car[NT];                // per run: the sum after its last row end
   unsigned ends[NT];         // per run: bit k set where its k-th nonzero ends a row
@@ -379,6 +379,7 @@ __device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, 
   const int p0 = tid * PER;
   const bool active = p0 < end;
   S.ends[tid] = 0u;
+  if (tid == 0) S.xs[RB_XCAP] = (XT)0;
   __syncthreads();
   // x at the distinct columns
 #pragma unroll
@@ -397,24 +398,17 @@ __device__ __forceinline__ void rb_compute(const RbCsr<VT> &M, RbRegs<VT, NNZB, 
     }
     __syncthreads();
     if (active) {
-      // a run with entries of a neighbouring block: they count as 0 times 0, whatever x is
-      const bool edge = p0 < d || p0 + PER > end;
-      if (edge) {
+      if (p0 < d || p0 + PER > end) {  // a run with entries of a neighbouring block: 0 times 0, whatever x is
 #pragma unroll
         for (int k = 0; k < PER; ++k)
           if (p0 + k < d || p0 + k >= end) {
             R.v[k] = (VT)0;
-            R.li[k] = 0;
+            R.li[k] = RB_XCAP;
           }
       }
       XT xv[PER];
 #pragma unroll
       for (int k = 0; k < PER; ++k) xv[k] = S.xs[R.li[k]];
-      if (edge) {
-#pragma unroll
-        for (int k = 0; k < PER; ++k)
-          if (p0 + k < d || p0 + k >= end) xv[k] = (XT)0;
-      }
       const unsigned m = S.ends[tid];
       int row = S.row[tid];
       XT s = (XT)0;
