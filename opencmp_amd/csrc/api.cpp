@@ -421,9 +421,11 @@ void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
   std::vector<int32_t> rblk;
   rblk.push_back(0);
   int64_t start_nz = 0;
+  int64_t live = A->n;  // rows behind the last nonzero have blocks of their own
+  while (live > 0 && A->row_ptr[live] == A->row_ptr[live - 1]) --live;
   for (int64_t r = 0; r < A->n; ++r) {
     const int64_t end_nz = A->row_ptr[r + 1];
-    if ((end_nz - start_nz > cap || r - rblk.back() >= RB_ROWS) && rblk.back() != r) {
+    if ((end_nz - start_nz > cap || r - rblk.back() >= RB_ROWS || r == live) && rblk.back() != r) {
       rblk.push_back((int32_t)r);
       start_nz = A->row_ptr[r];
     }
@@ -579,7 +581,16 @@ void build_solver_operator(Matrix *A) {
   }
   std::vector<int32_t> order(A->n);
   for (int64_t r = 0; r < A->n; ++r) order[r] = (int32_t)r;
-  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return key[a] < key[b]; });
+  // rows of which nothing is left come last: a row block among the others has none of them, which keeps it
+  // on the kernel's path of runs (P2 on 300^2 triangles with one of two components left out of the form,
+  // FP64: an FGMRES iteration 82 us with them in between, 62 now)
+  std::vector<uint8_t> none(A->n, 1);
+  for (int64_t r = 0; r < A->n; ++r)
+    for (int32_t k = A->row_ptr[r]; k < A->row_ptr[r + 1] && none[r]; ++k)
+      none[r] = !(A->active_pairs >> (blk[r] * nb + blk[A->col[k]]) & 1);
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+    return none[a] != none[b] ? none[a] < none[b] : key[a] < key[b];
+  });
   auto *M = new Matrix();
   M->space = A->space;
   M->ctx = A->ctx;

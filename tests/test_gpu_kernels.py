@@ -181,6 +181,35 @@ def test_spmv_rows_without_nonzeros(gpu_ctx, precision):
     assert rel(sol[0][:n], sol[1]) < 1e-10 and not sol[0][n:].any()
 
 
+# rows without nonzeros before, behind and between the others, whole blocks of them, blocks of 4096 nonzeros
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('make,order,live', [
+    (lambda: unit_square(1), 1, (0, 1)), (lambda: unit_square(12), 1, (1, 0, 0)), (lambda: unit_square(40), 2, (0, 1, 0)),
+    (lambda: unit_square(30), 3, (0, 0, 1)), (lambda: unit_cube(15), 3, (1, 0)),
+])
+def test_spmv_some_rows_without_nonzeros(gpu_ctx, make, order, live, precision):
+    """As above with the live component first, last or in the middle: the solution solves the system, by
+    scipy's product with the same matrix. The solver's residual is at most 1e-12 |f|; the two products
+    differ by the rounding of rows of at most 100 terms, below 100 * 1.1e-16 | |A| |u| |."""
+    C = core()
+    hm = make()
+    k = live.index(1)
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.H1(order if c else 1) for c in live])
+    a = C.BilinearForm(fes, [C.Vol('gradgrad', k, k, coef=1e-4), C.Vol('mass', k, k)])
+    f = C.LinearForm(fes, [C.Source(k, (L.FN_POLY2, POLY[hm.dim]))])
+    a.Assemble()
+    f.Assemble()
+    pre = C.Preconditioner(a, 'local', precision=precision)
+    pre.Update()
+    u = C.GridFunction(fes)
+    r = C.solve(a, f.vec, u.vec, pre, 'FGMRes', tol=1e-12, precision=precision, restart=60, inner_tol=1e-4)
+    assert r.converged
+    off = fes.block_offsets()
+    v, b, A = u.vec.cpu().numpy(), f.vec.cpu().numpy(), a.to_scipy()
+    assert not v[:off[k]].any() and not v[off[k + 1]:].any()
+    assert np.linalg.norm(b - A @ v) <= 1e-12 * np.linalg.norm(b) + 1.1e-14 * np.linalg.norm(abs(A) @ abs(v))
+
+
 # ------------------------------------------------------------------------------------------ row gather
 
 
