@@ -222,10 +222,15 @@ struct WGrads {
   WGrad l[NL];
 };
 
+// A chunk grows with the grid beyond 256 of them (from 53^3 voxels on): a wavefront's FP32 sums run over at most WG_RUN
+// tiles of 16 voxels and are then added up, so that a sum of 129^3 products is 128 + 17 additions long and
+// not 2,096; the partial sums of the chunks and the biases are summed in FP64.
+constexpr int WG_RUN = 8;
+
 __device__ __forceinline__ int64_t chunk_len(int64_t n, int nch) { return ((n + nch - 1) / nch + 15) / 16 * 16; }
 
 __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__ part) {
-  __shared__ float sh[4][9 * 256];
+  __shared__ alignas(16) float sh[4][9 * 256];
   int l = 0;
   while (l + 1 < NL && (int)blockIdx.x >= T.l[l + 1].blk0) ++l;
   const WGrad &g = T.l[l];
@@ -243,16 +248,16 @@ __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__
     const int64_t zg = (int64_t)g.ng * g.ng * g.ng, cl = chunk_len(zg, g.nch);
     const int64_t z0 = ch * cl, z1 = min(zg, z0 + cl);
     const int cch = ct * 16 + li;
-    float s = 0.f;
+    double s = 0.0;
     if (cch < g.nc)
-      for (int64_t z = z0 + wv * 4 + lk; z < z1; z += 16) s += ((const float *)g.G)[(int64_t)cch * zg + z];
-    sh[wv][lane] = s;
+      for (int64_t z = z0 + wv * 4 + lk; z < z1; z += 16) s += (double)((const float *)g.G)[(int64_t)cch * zg + z];
+    double *shd = reinterpret_cast<double *>(sh[0]);
+    shd[threadIdx.x] = s;
     __syncthreads();
     if (threadIdx.x < 16 && ct * 16 + (int)threadIdx.x < g.nc) {
-      float t = 0.f;
-      for (int w = 0; w < 4; ++w)
-        for (int k = 0; k < 4; ++k) t += sh[w][k * 16 + threadIdx.x];
-      out[(int64_t)g.na * g.nb * 27 + ct * 16 + threadIdx.x] = t;
+      double t = 0.0;
+      for (int k = 0; k < 16; ++k) t += shd[k * 16 + threadIdx.x];
+      out[(int64_t)g.na * g.nb * 27 + ct * 16 + threadIdx.x] = (float)t;
     }
     return;
   }
@@ -264,6 +269,18 @@ __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__
   f32x4 acc[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int run = 0;
+  bool more = false;
+  auto put = [&]() {  // to the wavefront's own part of LDS
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float &t = sh[wv][k * 256 + r * 64 + lane];
+        t = more ? t + acc[k][r] : acc[k][r];
+      }
+    more = true;
+  };
   // the 40 loads of four voxels go out together: what lies outside reads the channel's first value and counts 0
   auto sweep = [&](auto *P, auto *Q) {
     for (int64_t zb = z0 + wv * 16; zb < z1; zb += 64) {
@@ -298,6 +315,12 @@ __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int k = 0; k < 9; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[r], qv[r][k], acc[k], 0, 0, 0);
+      if (++run == WG_RUN && zb + 64 < z1) {
+        run = 0;
+        put();
+#pragma unroll
+        for (int k = 0; k < 9; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
     }
   };
   if (g.p_bf16) {
@@ -311,10 +334,7 @@ __global__ __launch_bounds__(NT) void k_conv_wgrad(WGrads T, float *__restrict__
     else
       sweep((const float *)g.P, (const float *)g.Q);
   }
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sh[wv][k * 256 + r * 64 + lane] = acc[k][r];
+  put();
   __syncthreads();
   const int t = threadIdx.x;
   const int ao = ta * 16 + 4 * ((t & 63) >> 4) + (t >> 6), bo = tb * 16 + (t & 15);
@@ -334,9 +354,10 @@ __global__ void k_chunk_reduce(WGrads T, const float *__restrict__ part, float *
   const WGrad &g = T.l[l];
   const int64_t len = (int64_t)g.na * g.nb * 27 + g.nc;
   const float *__restrict__ p = part + g.part + (j - g.off);
-  float s = 0.f;
-  for (int c = 0; c < g.nch; ++c) s += p[(int64_t)c * len];
-  grad[j] = accumulate ? grad[j] + s : s;
+  double s = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < g.nch; ++c) s += (double)p[(int64_t)c * len];
+  grad[j] = accumulate ? grad[j] + (float)s : (float)s;
 }
 
 __global__ void k_adam_step(int n, const float *__restrict__ grad, float gscale, float *p, float *m, float *v,
@@ -540,7 +561,8 @@ static void unet_forward(Unet *U, hipStream_t st) {
 }
 
 // what every layer's parameter gradient is formed from, and the partition of its voxels: chunks of
-// 512 voxels (a wavefront's share keeps its nine accumulators busy for eight tiles) and at most 256
+// 512 voxels (a wavefront's share keeps its nine accumulators busy for eight tiles), longer on grids that
+// would give more than 256
 static WGrads wgrad_table(Unet *U, int64_t *part_len, int *nblocks) {
   WGrads T;
   int64_t po = 0;

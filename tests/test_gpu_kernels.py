@@ -365,6 +365,40 @@ def test_unet_tiles(gpu_ctx, N):
             o += size
 
 
+def test_unet_gradient_of_a_large_grid(gpu_ctx):
+    """Sums over 129^3 voxels, known exactly: all weights zero, the last hidden layer's bias 1, so that the
+    last layer's weight gradient is the output gradient summed over the voxels that a tap reaches, and its
+    bias gradient over all. Constant output gradients let every rounding of a long FP32 sum fall on the
+    same side. FP32 sums of 128 products and of 17 such sums, four wavefronts, FP64 beyond and one rounding:
+    at most (128 + 17 + 2 + 1) 2^-24 relative."""
+    import torch
+    from opencmp_amd.learned import UNetPrecond
+    from oracle import unet as ou
+    N = 128
+    n = N + 1
+    p = {k: np.zeros_like(v) for k, v in ou.unpack(np.zeros(ou.NPARAM, np.float32)).items()}
+    flat, o, at = np.zeros(ou.NPARAM, np.float32), 0, {}
+    for name, kind, ci, co, s in ou.LAYERS:
+        at[name] = (o, o + ci * co * 27, o + ci * co * 27 + co)
+        o = at[name][2]
+    assert o == ou.NPARAM and set(p) == {f'{k}.{w}' for k in at for w in 'Wb'}
+    hidden, last = ou.LAYERS[6][0], ou.LAYERS[7][0]
+    flat[at[hidden][1]:at[hidden][2]] = 1.0
+    c = np.array([1.167053, 1.8018806, 1.0147063, 1.6719949], np.float32)
+    U = UNetPrecond(N, gpu_ctx, params=flat)
+    x = torch.zeros((4, n ** 3), device='cuda')
+    gy = torch.from_numpy(c).cuda().reshape(4, 1).expand(4, n ** 3).contiguous()
+    g = U.grad(x, gy).cpu().numpy().astype(np.float64)
+    d = np.array([n - 1, n, n - 1], np.float64)     # voxels that a tap of -1, 0, 1 reaches along an axis
+    taps = np.einsum('i,j,k->ijk', d, d, d).ravel()
+    ci, co = ou.LAYERS[7][2], ou.LAYERS[7][3]
+    W = g[at[last][0]:at[last][1]].reshape(co, ci, 27)
+    ref = c.astype(np.float64)[:, None, None] * taps
+    assert np.abs(W / ref - 1.0).max() <= 148 * 2.0 ** -24
+    b = g[at[last][1]:at[last][2]]
+    assert np.abs(b / (c.astype(np.float64) * n ** 3) - 1.0).max() <= 148 * 2.0 ** -24
+
+
 # ------------------------------------------------------------------------------------------ MLP tiles
 
 
