@@ -3902,9 +3902,13 @@ static int fgmres_cycle(Matrix *A, Matrix *K, Precond *P, bool learned, const do
   int j = 0, bidx = 0, k_used = -1;
   // inner solve (Schur PCG, or the velocity PCG of the block-triangular step) with a tolerance:
   // each step enqueues `cap` iterations (the rest of a converged inner solve are empty launches);
-  // after each batch the host reads how many ran and sets the cap to 1.1x that plus 4 (the count
-  // changes by a few from step to step: with 1.3x plus 10 half of the launches of a 3D diffuse-interface
-  // Stokes solve were empty, at 2.3 us each), doubling it when a step used them all
+  // after each batch the host reads how many ran and sets the cap to that plus some room, doubling it
+  // when a step used them all. Room for the velocity PCG is a tenth plus 4: its counts change by a few from
+  // step to step, and the outer iterations of 3D diffuse-interface Stokes (6^3 to 14^3, six inputs each)
+  // are those with three tenths plus 10, which leaves half of the launches empty at 2.3 us each (14^3
+  // mixed: 44.1 ms a solve against 46.5). The counts of the Schur PCG jump more, and a step cut short costs
+  // outer iterations: six start-up steps of the channel at n = 114, mixed, take 2,351 with three tenths plus
+  // 10 (1.62 s) and 2,490 with a tenth plus 4 (1.66 s)
   const bool btri = P->btri;
   const int in_iters = btri ? P->vel_iters : P->schur_iters;
   const bool adapt = in_iters > 0 && (btri ? P->vel_tol : P->schur_tol) > 0.0;
@@ -3996,7 +4000,8 @@ static int fgmres_cycle(Matrix *A, Matrix *K, Precond *P, bool learned, const do
       const double cnt = hres[m + 2 + b.ev];
       const double per = (cnt - in_seen) / nb_run;
       in_seen = cnt;
-      in_cap = per >= b.cap - 0.5 ? std::min(in_iters, 2 * b.cap) : std::min(in_iters, (int)(1.1 * per) + 4);
+      const int room = btri ? (int)(1.1 * per) + 4 : (int)(1.3 * per) + 10;
+      in_cap = std::min(in_iters, per >= b.cap - 0.5 ? 2 * b.cap : room);
     }
     if (conv >= 0) k_used = b.j0 + conv + 1;
   }

@@ -509,6 +509,36 @@ def test_s_step_blocks(gpu_ctx, n, precision):
     assert float(r.norm()) <= 1.01e-9 * float(f.vec.norm())
 
 
+def test_inner_iteration_cap_costs_few_outer_iterations(gpu_ctx):
+    """The Schur PCG's launches of a step are capped by the counts of the steps before. In one cycle of the
+    two Stokes steps here FGMRES takes 109 and 102 iterations without a cap (one batch for the whole cycle,
+    so no count is known in it); caps with three tenths plus ten of room take 111 and 107, with a tenth plus
+    four 118 and 115. Half of the way between the sums, 6 % more than without a cap, is allowed."""
+    C = core()
+    from opencmp_amd.models import Stokes, const
+    inflow = [(L.FN_POLY2, [0, 0, 4.0, 0, 0, -4.0]), const(0.0)]
+    wall = [const(0.0), const(0.0)]
+    its = {1: 0, 150: 0}
+    for n, dt in ((16, 1e-2), (32, 1e-3)):
+        m = Stokes(unit_square(n), kv=1.0, interp_ord=2, dirichlet={'u': {'left': inflow, 'top': wall, 'bottom': wall}},
+                   linear_solver='GMRes', preconditioner='schur', linear_tolerance=1e-10, restart=150,
+                   schur_iters=200, schur_tol=0.1, ctx=gpu_ctx)
+        a = C.BilinearForm(m.fes, m.time_derivative_terms() + m.construct_bilinear_time_coefficient(dt) +
+                           m.construct_bilinear_time_ODE(dt))
+        f = C.LinearForm(m.fes, m.construct_linear(dt))
+        a.Assemble()
+        f.Assemble()
+        for check in its:
+            pre = m.construct_preconditioners(a)
+            pre.Update()
+            x = C.GridFunction(m.fes)
+            m.apply_dirichlet_bcs_to(x)
+            r = C.solve(a, f.vec, x.vec, pre, 'FGMRes', tol=1e-8, restart=150, maxit=150, check_every=check)
+            assert r.converged and r.outer == 1
+            its[check] += r.iters
+    assert its[1] <= 1.06 * its[150]
+
+
 def test_kept_plans_follow_the_form(gpu_ctx):
     """A form assembled again takes the coefficients, sources and field values of the moment, also after
     another form of the same space was assembled in between."""
