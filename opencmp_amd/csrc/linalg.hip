@@ -2782,7 +2782,7 @@ constexpr int CA_KQ_MAX = 16;
 // at condition ~1e4 instead of ~1e7 for plain powers (small enough for FP32 storage).
 constexpr double CA_SIGMA = 1.0;
 constexpr int CA_NG = CA_S * (CA_S + 1) / 2;
-constexpr int CA_FAC_BLOCKS = 1024;
+constexpr int CA_FAC_BLOCKS = 864;
 // largest restart of an s-step cycle: the block kernels size their LDS for k + 1 + CA_S <= CA_MMAX + 1
 // basis rows (the host only takes the s-step path for m <= CA_MMAX)
 constexpr int CA_MMAX = 50;
@@ -3042,8 +3042,8 @@ __device__ __forceinline__ void ca_factor_block(const double *__restrict__ gpart
   __syncthreads();
 }
 
-// The Gram matrix' partials summed and factored in one launch of one block, a wave an entry (768 partials:
-// 6.1 us; a launch to sum and one to factor before: 4.5 + 4.2 us)
+// The Gram matrix' partials summed and factored in one launch of one block, a wave an entry (1,024 partials: 7.5
+// us; 768: 6.1, where a launch to sum and one to factor took 4.5 + 4.2 us)
 __global__ void __launch_bounds__(1024) k_ca_chol(const double *__restrict__ gpart, int np, double *__restrict__ R,
                                                   double *__restrict__ Rinv, double *__restrict__ flag) {
   __shared__ double gs[CA_NG], Rl[CA_S * CA_S], Ri[CA_S * CA_S];
@@ -3213,7 +3213,8 @@ __device__ __forceinline__ void ca_hess(const CaHess &h, CaHessLds &l, const dou
 // factor is not ready, every block sums the Gram partials (np per entry) and factors for itself;
 // block 0 stores R. All of it is latency: sum, factor and solve, twice, and the columns were seven launches of 2.8,
 // 3.0, 3.8 and once 7.0 us on 27,648 FP64 unknowns with their gaps, now two of 7.0 us (DG-P2 48^2: 15.1 -> 11.8 ms a solve);
-// 786,432 FP32 unknowns: 4.5 + 4.2 + 6.9 + 8.5 us -> 9.8 us after a k_ca_chol of 6.1 (256^2: 150.9 -> 140.7 ms).
+// 786,432 FP32 unknowns: 4.5 + 4.2 + 6.9 + 8.5 us -> 15.3 us (256^2: 150.9 -> 140.7 ms); 1,306,800, with a
+// k_ca_chol of 7.5 us before it: 12.6 us.
 struct CaFactor {
   const double *gpart;
   int np;
@@ -3351,9 +3352,11 @@ static int ca_gmres_cycle(Matrix *A, Precond *P, const double *r0, double beta, 
   const size_t npc = (size_t)(m + 1) * CA_S * dgrid;
   ensure_part(w, std::max((size_t)(m + 1) * CA_S * grid + 64, npc + 2 * (size_t)CA_NG * grid));
   double *gp1 = w.part.p + npc, *gp2 = gp1 + (size_t)CA_NG * grid;
-  // every block of the triangular solve factors for itself up to CA_FAC_BLOCKS partials an entry: DG-P2 96^2
-  // FP64 (216 partials) 21.0 ms a solve against 21.9 with a launch for it, 200^2 FP32 (472) 76.4 against 77.2,
-  // 256^2 FP32 (768) 140.7 against 141.4; beyond, each block would read more for it than of its rows
+  // every block of the triangular solve factors for itself up to CA_FAC_BLOCKS partials an entry; beyond, each
+  // would read more for it than of its rows, and a launch of one block does it (the grid ends at
+  // STREAM_BLOCKS). An iteration with the one and the other, DG-P2 FP64: 756 partials 27.4 and 27.6 us, 888
+  // 32.1 and 32.0, 984 35.0 and 34.4, 1024 41.8 and 40.9; FP32: 768 26.9 and 27.1 us, 864 30.6 and 30.6, 968 32.6
+  // and 32.6, 1024 40.1 and 39.8
   const bool fac = grid <= CA_FAC_BLOCKS;
   k_scale_copy<double, T><<<nblk(n), NTHR, 0, st>>>(n, r0, 1.0 / beta, Q);
   // g = e_0 (relative to beta), flag = 0, one = 1

@@ -487,8 +487,9 @@ def test_cg_forms(gpu_ctx, n, precision):
     assert float(r.norm()) <= 1.01 * tol * float(b.norm()) + 1e-15 * 40 * float(u.vec.norm())
 
 
-# the s-step factor made by every block (up to 1024 Gram partials an entry) and in its own launch
-@pytest.mark.parametrize('n,precision', [(2, 'fp64'), (17, 'fp64'), (17, 'mixed'), (216, 'fp64')])
+# the s-step factor made by every block (up to 864 Gram partials an entry: 192^2 FP64) and in its own launch
+@pytest.mark.parametrize('n,precision', [(2, 'fp64'), (17, 'fp64'), (17, 'mixed'), (192, 'fp64'), (193, 'fp64'),
+                                         (216, 'fp64'), (300, 'mixed')])
 def test_s_step_blocks(gpu_ctx, n, precision):
     import torch
     C = core()
