@@ -3056,12 +3056,8 @@ __global__ void __launch_bounds__(1024) k_ca_chol(const double *__restrict__ gpa
   if (threadIdx.x == 0 && !ok) flag[0] = 1.0;
 }
 
-// New Hessenberg columns k..k+S-1 from the change of basis (Ahat v_t = v_{t+1} + d_t v_t -
-// c_t v_{t-1}), then their Givens rotations.
-// Hf: unrotated Hessenberg, Hr: rotated (both column-major, ld = m+1). C: (k+1) x S q-major.
-// The residual estimates of the new columns and the CholQR breakdown flag also go straight to the
-// host's pinned status buffer hst (res at [j], the flag at [m + 8 + slot]); the host reads them
-// after the event recorded behind this kernel.
+// what the new Hessenberg columns of a block are made from; Hf: unrotated Hessenberg, G.R: rotated (both
+// column-major, ld = m+1); C: (k+1) x S, q-major
 struct CaHess {
   int on, k, m, slot;
   const double *C, *R1, *R2;  // R1, R2: the factors of the first and second pass; R2 is null after a single pass
@@ -3094,6 +3090,11 @@ __device__ __forceinline__ void ca_hess_load(const CaHess &h, CaHessLds &l, doub
   for (int e = tid; e < (k + 1) * CA_S; e += blockDim.x) l.Rr[(e % CA_S + 1) * nr + e / CA_S] = h.C[e];
   for (int e = tid; e < nr; e += blockDim.x) l.Rr[e] = e == k ? 1.0 : 0.0;
 }
+// New Hessenberg columns k..k+S-1 from the change of basis (Ahat v_t = v_{t+1} + d_t v_t -
+// c_t v_{t-1}), then their Givens rotations.
+// The residual estimates of the new columns and the CholQR breakdown flag also go straight to the
+// host's pinned status buffer hst (res at [j], the flag at [m + 8 + slot]); the host reads them
+// after the event recorded behind this launch.
 __device__ __forceinline__ void ca_hess(const CaHess &h, CaHessLds &l, const double (&hr)[CA_HT], const double *R1,
                                         const double *R2, bool broken) {
   const int k = h.k, m = h.m, ld = m + 1, nr = k + 1 + CA_S;
@@ -3205,8 +3206,6 @@ __device__ __forceinline__ void ca_hess(const CaHess &h, CaHessLds &l, const dou
   hst[m + 8 + h.slot] = broken ? 1.0 : 0.0;
 }
 
-// One CA-GMRES(m) cycle on the DG operator Ahat (block Jacobi folded in); same contract as
-// gmres_cycle. Returns -1 (and changes nothing in x) if the first block breaks down.
 // W <- W R^{-1} (R upper triangular S x S, row-major), Gram partials of the result if part.
 // The first NXCD blocks of the grid carry no rows (so that the others keep their place on the XCDs):
 // block 0 does the block's Hessenberg columns meanwhile, which need the factor and not W. FAC: the
@@ -3318,6 +3317,8 @@ __global__ void __launch_bounds__(NTHR) k_btrsm_gram(int64_t n, T *__restrict__ 
   block_sums<CA_NG + 1>(v, sh, CA_NG, part + lb, nb);
 }
 
+// One CA-GMRES(m) cycle on the DG operator Ahat (block Jacobi folded in); same contract as
+// gmres_cycle. Returns -1 (and changes nothing in x) if the first block breaks down.
 template <typename T>
 static int ca_gmres_cycle(Matrix *A, Precond *P, const double *r0, double beta, double *x, int m, double stop_abs,
                           int maxit, Work &w, bool &breakdown, CaShift &shift, bool &newton) {
