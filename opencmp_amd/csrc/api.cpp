@@ -411,7 +411,7 @@ void build_pattern(Matrix *A) {
   A->d_col.upload(A->col, st);
   A->d_val.alloc(A->nnz);
   OCMP_HIP(hipMemsetAsync(A->d_val.p, 0, A->nnz * sizeof(double), st));
-  build_row_blocks(A, A->rb, spmv_nnzb(A->nnz));
+  build_row_blocks(A, A->rb, spmv_nnzb(A->n, A->nnz));
 }
 
 void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
@@ -613,7 +613,7 @@ void build_solver_operator(Matrix *A) {
   M->d_src.upload(src.empty() ? std::vector<int32_t>(1, 0) : src, st);
   M->d_rowmap.upload(order, st);
   M->d_val.alloc(std::max<int64_t>(M->nnz, 1));
-  build_row_blocks(M, M->rb, spmv_nnzb(M->nnz));
+  build_row_blocks(M, M->rb, spmv_nnzb(M->n, M->nnz));
   M->assembled = true;
   OCMP_HIP(hipStreamSynchronize(st));
   delete A->op;
@@ -1242,7 +1242,7 @@ void build_velocity_blocks(Precond *P) {
     M->d_row_ptr.upload(M->row_ptr, st);
     M->d_col.upload(M->col, st);
     M->d_val.alloc(M->nnz);
-    build_row_blocks(M, M->rb, spmv_nnzb(M->nnz));
+    build_row_blocks(M, M->rb, spmv_nnzb(M->n, M->nnz));
     M->assembled = true;
     return M;
   };

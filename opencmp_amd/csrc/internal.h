@@ -293,7 +293,7 @@ struct Matrix {
   DBuf<int8_t> d_dg_pos;             // nel*(dim+2): pos of diag block, then of each facet neighbour (-1 none)
   DBuf<int32_t> d_dg_bcol;           // nel*4 block columns (-1 padded), sorted
   int dg_nb = 0;                     // local dofs per element (block size)
-  RowBlocks rb;  // row blocks of the LDS-staged SpMV, of spmv_nnzb(nnz) nonzeros
+  RowBlocks rb;  // row blocks of the LDS-staged SpMV, of spmv_nnzb nonzeros
   bool assembled = false;
   // mixed precision copy
   DBuf<float> d_val32;
@@ -477,12 +477,18 @@ void build_h1_schedule(Matrix *A);
 void build_h1_gather(Matrix *A);
 void build_colouring(Space &s);
 void build_pattern(Matrix *A);
-// nonzeros per row block of the LDS-staged SpMV: large blocks where there are enough of them for
-// several a CU (62M FP64 nonzeros: 157 us against 169 with small ones), small ones below, where one
-// block's chain of loads and sums is the launch's time
+// Nonzeros per row block of the LDS-staged SpMV: large blocks where there are enough of them for several a
+// CU, small ones below, where one block's chain of loads and sums is the launch's time. The line is lower
+// for rows of more than 24 nonzeros, where a block has fewer rows to sum. FP64 products, small and large
+// blocks: 1.4M nonzeros of 3D P3 6.0 and 6.2 us, 2.5M of 3D P2 7.2 and 7.3, 3.7M of 3D P2 13.2 and 10.8, of 3D
+// P3 14.7 and 10.7, 62M 169 and 157. FP32 CG iterations on short rows, 2D P2: 3.7M 23.6 and 25.9 us, 6M 30.9 and
+// 34.6, 12M 43.5 and 47.9; on 3D P1 (15 a row): 3.7M 20.8 and 21.2, 6.2M 28.6 and 26.3.
 constexpr int SPMV_NNZB = 2048, SPMV_NNZB_LARGE = 4096;
-constexpr int64_t SPMV_LARGE_NNZ = (int64_t)4 << 20;
-inline int spmv_nnzb(int64_t nnz) { return nnz >= SPMV_LARGE_NNZ ? SPMV_NNZB_LARGE : SPMV_NNZB; }
+constexpr int64_t SPMV_LARGE_NNZ = (int64_t)4 << 20, SPMV_LARGE_NNZ_LONG = (int64_t)3 << 20;
+constexpr int SPMV_LONG_ROW = 24;
+inline int spmv_nnzb(int64_t n, int64_t nnz) {
+  return nnz >= (nnz >= SPMV_LONG_ROW * n ? SPMV_LARGE_NNZ_LONG : SPMV_LARGE_NNZ) ? SPMV_NNZB_LARGE : SPMV_NNZB;
+}
 // the fused Schur PCG iteration: row blocks of S of this many nonzeros, SCG_NT threads a block
 constexpr int SCG_NNZB = 4096;
 constexpr int SCG_NT = 512;

@@ -107,6 +107,7 @@ def shuffled(m, seed):
     ('one block', lambda: unit_square(1), 1),
     ('several small blocks', lambda: unit_square(23), 3),
     ('large blocks', lambda: unit_cube(15), 3),
+    ('large blocks of long rows', lambda: unit_cube(14), 3),
     ('rows of 4,503 nonzeros', lambda: fan(250), (3, 3)),
     ('rows of 2,042 nonzeros, longer than a block', lambda: fan(170), (3, 2)),
     ('rows of 2,030 nonzeros, each a block', lambda: fan(169), (3, 2)),
