@@ -414,6 +414,24 @@ void build_pattern(Matrix *A) {
   build_row_blocks(A, A->rb, spmv_nnzb(A->n, A->nnz));
 }
 
+// Per thread an array with a number for every column, of which a thread uses few and neighbouring ones at a
+// time unless the mesh is numbered at random (then it is walked all over). Left to the system to zero when
+// a page is first touched; as many threads as find room in COLPOS_BYTES. (A hash table of a few
+// thousand columns a thread took twice the time on meshes in order, and as long on others.)
+constexpr int64_t COLPOS_BYTES = (int64_t)1 << 30;
+struct ColPos {
+  int nt;
+  std::vector<std::unique_ptr<int32_t, void (*)(void *)>> p;
+  explicit ColPos(int64_t ncol) {
+    ncol = std::max<int64_t>(ncol, 1);
+    nt = (int)std::max<int64_t>(1, std::min<int64_t>(omp_get_max_threads(), COLPOS_BYTES / (ncol * 4)));
+    for (int t = 0; t < nt; ++t) {
+      p.emplace_back((int32_t *)std::calloc(ncol, sizeof(int32_t)), std::free);
+      if (!p.back()) throw std::bad_alloc();
+    }
+  }
+};
+
 void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
   // greedy: extend a block while its nonzeros and rows fit; a row longer than that is a block of
   // its own (the kernel then loops over it in chunks and keeps global columns)
@@ -437,8 +455,10 @@ void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
   int32_t cmax = -1;
 #pragma omp parallel for schedule(static) reduction(max : cmax)
   for (int64_t j = 0; j < A->nnz; ++j) cmax = std::max(cmax, A->col[j]);
-  const int64_t ncol = (int64_t)cmax + 1;  // transfers between levels are not square
-  std::vector<uint16_t> lcol(A->nnz);
+  const ColPos pos((int64_t)cmax + 1);  // transfers between levels are not square
+  // (large arrays here and below are left to the threads to touch first: cleared by one, their pages
+  // were a third of the time)
+  const std::unique_ptr<uint16_t[]> lcol(new uint16_t[std::max<int64_t>(A->nnz, 1)]);
   std::vector<std::vector<int32_t>> ub;
   std::vector<uint8_t> done;  // blocks whose list is built
   for (;;) {
@@ -449,46 +469,39 @@ void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
     }
     std::vector<uint8_t> over(nb, 0);
     bool any = false;
-    // per thread and column: the last block of the thread that has it, and its position in that
-    // block's list. Zeroed lazily by the system: a thread's blocks are consecutive and touch few pages.
-    struct Col {
-      int32_t blk, pos;
-    };
-    std::vector<std::unique_ptr<Col, void (*)(void *)>> seen;
-    for (int t = 0; t < omp_get_max_threads(); ++t) {
-      seen.emplace_back((Col *)std::calloc(std::max<int64_t>(ncol, 1), sizeof(Col)), std::free);
-      if (!seen.back()) throw std::bad_alloc();
-    }
-#pragma omp parallel
+#pragma omp parallel num_threads(pos.nt)
     {
-      Col *const col_of = seen[omp_get_thread_num()].get();
+      // a column's position in the block's list; it is in the list if it stands there
+      int32_t *const at = pos.p[omp_get_thread_num()].get();
       std::vector<int32_t> buf;
-      int32_t id = 0;
 #pragma omp for schedule(static) reduction(|| : any)
       for (int64_t b = 0; b < nb; ++b) {
         if (done[b]) continue;
         done[b] = 1;
         const int64_t j0 = A->row_ptr[rblk[b]], j1 = A->row_ptr[rblk[b + 1]];
-        if (j1 - j0 > cap) continue;
-        ++id;
+        if (j1 - j0 > cap) {
+          std::fill(lcol.get() + j0, lcol.get() + j1, 0);
+          continue;
+        }
         buf.clear();
-        for (int64_t j = j0; j < j1; ++j) {
-          Col &c = col_of[A->col[j]];
-          if (c.blk != id) {
-            c.blk = id;
-            buf.push_back(A->col[j]);
-          }
+        for (int64_t j = j0; j < j1 && (int64_t)buf.size() <= RB_XCAP; ++j) {
+          const int32_t c = A->col[j], p = at[c];
+          if (p < (int32_t)buf.size() && buf[p] == c) continue;
+          at[c] = (int32_t)buf.size();
+          buf.push_back(c);
         }
         if ((int64_t)buf.size() > RB_XCAP) {
           if (rblk[b + 1] - rblk[b] > 1) {
             over[b] = 1;
             any = true;
+          } else {
+            std::fill(lcol.get() + j0, lcol.get() + j1, 0);
           }
           continue;
         }
         std::sort(buf.begin(), buf.end());
-        for (size_t i = 0; i < buf.size(); ++i) col_of[buf[i]].pos = (int32_t)i;
-        for (int64_t j = j0; j < j1; ++j) lcol[j] = (uint16_t)col_of[A->col[j]].pos;
+        for (size_t i = 0; i < buf.size(); ++i) at[buf[i]] = (int32_t)i;
+        for (int64_t j = j0; j < j1; ++j) lcol[j] = (uint16_t)at[A->col[j]];
         ub[b] = buf;
       }
     }
@@ -528,7 +541,7 @@ void build_row_blocks(Matrix *A, RowBlocks &rb, int nnzb) {
   rb.nucol = nu[nb];
   rb.d_desc.upload(desc, A->ctx->stream);
   rb.d_ucol.upload(ucol, A->ctx->stream);
-  rb.d_lcol.upload(lcol, A->ctx->stream);
+  rb.d_lcol.upload(lcol.get(), A->nnz, A->ctx->stream);
   rb.nnzb = nnzb;
 }
 
@@ -1364,7 +1377,7 @@ void build_h1_gather(Matrix *A) {
   const int64_t nblk = (int64_t)gblk.size() - 1;
   // per block: entries sorted by local row (stable), and for every nonzero the staged values it sums,
   // in the rows' element order
-  std::vector<int32_t> spe(np);
+  const std::unique_ptr<int32_t[]> spe(new int32_t[std::max<int64_t>(np, 1)]);
   std::vector<GatherBlk> desc(nblk);
   int64_t ix8 = 0;
   for (int64_t b = 0; b < nblk; ++b) {
@@ -1374,23 +1387,21 @@ void build_h1_gather(Matrix *A) {
     ix8 += ((int64_t)desc[b].ne * nl + 7) / 8;
   }
   OCMP_REQUIRE(ix8 < INT32_MAX, "too many element entries");
-  std::vector<uint16_t> gend(A->nnz), gidx((size_t)ix8 * 8, 0);
+  const std::unique_ptr<uint16_t[]> gend(new uint16_t[std::max<int64_t>(A->nnz, 1)]);
+  const std::unique_ptr<uint16_t[]> gidx(new uint16_t[std::max<int64_t>(ix8, 1) * 8]);
   std::vector<std::vector<uint32_t>> units(nblk);
-  std::vector<std::unique_ptr<int32_t, void (*)(void *)>> pos_of;  // per thread: a row's column -> its position
-  for (int t = 0; t < omp_get_max_threads(); ++t) {
-    pos_of.emplace_back((int32_t *)std::malloc(std::max<int64_t>(n, 1) * sizeof(int32_t)), std::free);
-    if (!pos_of.back()) throw std::bad_alloc();
-  }
-#pragma omp parallel
+  const ColPos pos_of(n);  // a row's column -> its position
+#pragma omp parallel num_threads(pos_of.nt)
   {
-    int32_t *const pos = pos_of[omp_get_thread_num()].get();
+    int32_t *const pos = pos_of.p[omp_get_thread_num()].get();
     std::vector<int> cnt, fill;
     std::vector<int32_t> zof, start;
 #pragma omp for schedule(static)
     for (int64_t b = 0; b < nblk; ++b) {
       const int32_t r0 = gblk[b], r1 = gblk[b + 1];
       const int32_t e0 = desc[b].e0, ne = desc[b].ne, z0 = desc[b].z0, nz = desc[b].nz;
-      uint16_t *const ix = gidx.data() + (size_t)desc[b].ix8 * 8;
+      uint16_t *const ix = gidx.get() + (size_t)desc[b].ix8 * 8;
+      for (int64_t k = (int64_t)ne * nl; k & 7; ++k) ix[k] = 0;
       cnt.assign(nl + 1, 0);
       for (int32_t k = 0; k < ne; ++k) cnt[pli[e0 + k] + 1]++;
       for (int L = 0; L < nl; ++L) cnt[L + 1] += cnt[L];
@@ -1433,9 +1444,9 @@ void build_h1_gather(Matrix *A) {
   A->ngblk = nblk;
   A->d_gunit.upload(gunit, st);
   A->d_gblk.upload(desc, st);
-  A->d_pe.upload(spe, st);
-  A->d_gend.upload(gend, st);
-  A->d_gidx.upload(gidx, st);
+  A->d_pe.upload(spe.get(), np, st);
+  A->d_gend.upload(gend.get(), A->nnz, st);
+  A->d_gidx.upload(gidx.get(), (size_t)ix8 * 8, st);
   OCMP_HIP(hipStreamSynchronize(st));
 }
 
