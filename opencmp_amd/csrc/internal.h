@@ -188,8 +188,7 @@ struct Space {
   // load vectors (H1): per dof its entries among the element values (local dof * nel + element,
   // increasing) and the values (nloc x nel) they are summed from, built on first use; the kernels
   // of one space all run on its context's stream
-  DBuf<uint32_t> d_lptr;  // ndof+1
-  DBuf<uint32_t> d_lent;  // nel*nloc
+  DBuf<uint32_t> d_lidx;  // where a dof's entries start (ndof+1), the entries (nel*nloc), scratch
   DBuf<double> d_lin;     // nloc*nel
   std::map<std::string, std::string> lin_plans;  // load vectors: kernel arguments by terms and fields
   // cached kernel tables keyed by a signature
