@@ -2448,10 +2448,13 @@ void precond_update_jacobi(Precond *P) {
 // Batches of `check` iterations are enqueued ahead; the host checks the
 // residual history of batch b while batch b+1 runs, so the GPU never idles.
 //
-// Up to CG_SMALL_BLOCKS row blocks the small form (two launches an iteration; a launch there takes
-// its latency, and its blocks sum each other's few partials); above it the product gathers p alone, and
-// up to CG_SUM_BLOCKS partials of p.q the update sums them itself. 4,225 rows FP64: 24 -> 13.4 us an
-// iteration; 912k rows of 3D P3 in FP32: 94 -> 84 us.
+// Up to CG_SMALL_BLOCKS row blocks of SPMV_NNZB nonzeros (k_cg_spmv knows no other) the small form: two
+// launches an iteration; a launch there takes its latency, and its blocks sum each other's few partials.
+// Above it the product gathers p alone, and up to CG_SUM_BLOCKS partials of p.q the update sums them
+// itself. 4,225 rows FP64: 24 -> 13.4 us an iteration; 912k rows of 3D P3 in FP32: 94 -> 84 us. The small and the
+// other form near the line, FP64 (and FP32): 443 row blocks of 2D P2 14.3 and 15.8 us (13.7 and 15.3), 542 15.8
+// and 16.3 (14.6 and 15.8), 903 19.4 and 18.7 (16.5 and 16.9), 1,526 30.0 and 25.8; of 3D P3 486 13.8 and 15.3 (14.2
+// and 16.1), 882 16.5 and 16.7, 1,450 24.5 and 19.8: even at about 900, so the line is 3 to 8 % early.
 constexpr int CG_SMALL_BLOCKS = 512, CG_SUM_BLOCKS = 2048;
 template <typename VT, typename T>
 static int cg_inner(Matrix *A, const VT *val, const T *dinv, T *x, T *r, T *z, T *p, T *q, T *p2, double tol_rr,
@@ -2461,7 +2464,7 @@ static int cg_inner(Matrix *A, const VT *val, const T *dinv, T *x, T *r, T *z, T
   hipStream_t st = ctx->stream;
   const int64_t n = A->n;
   const int sgrid = spmv_grid<VT, T>(A);
-  const bool small = sgrid <= CG_SMALL_BLOCKS;
+  const bool small = sgrid <= CG_SMALL_BLOCKS && A->rb.nnzb == SPMV_NNZB;
   const int vgrid = std::min(red_grid(n), small ? 256 : 1024);
   ensure_part(w, (size_t)sgrid + SEG_BLOCKS + 64 + 2 * vgrid);
   double *pqpart = w.part.p, *vpart = w.part.p + sgrid + SEG_BLOCKS + 64;
