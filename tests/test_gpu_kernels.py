@@ -219,7 +219,7 @@ def test_spmv_some_rows_without_nonzeros(gpu_ctx, make, order, live, precision):
     (lambda: fan(16), 3),     # exactly one unit of 16 entries for the centre's row
     (lambda: fan(17), 2),     # and one entry more
     (lambda: fan(200), 3),    # a block grown to one row's 200 entries
-    (lambda: fan(250), 3),    # more than LDS takes: the element scatter
+    (lambda: fan(250), 3),    # and to 250: 33 KB of LDS
 ])
 def test_gather_units(gpu_ctx, make, order):
     """Matrix values against the oracle's quadrature, written, accumulated in a second launch (33 terms)
@@ -239,7 +239,7 @@ def test_gather_units(gpu_ctx, make, order):
 
     def gpu(terms):
         a = C.BilinearForm(fes, terms)
-        a.Assemble()
+        assert 'assemble_h1_gather' in _timed(gpu_ctx, a.Assemble)
         return a.values()
 
     G, M, X = (lambda c: C.Vol('gradgrad', 0, 0, coef=c)), (lambda c: C.Vol('mass', 0, 0, coef=c)), \
@@ -248,6 +248,34 @@ def test_gather_units(gpu_ctx, make, order):
     assert rel(gpu([G(2.0), G(2.0), M(0.5), X(0.5)]), ref(4.0, 0.5, 0.5)) < 1e-13
     assert rel(gpu([G(2.0), G(1.0), M(0.5), X(0.25)]), ref(3.0, 0.5, 0.25)) < 1e-13
     assert rel(gpu([G(1.0)] * 31 + [M(1.0), X(1.0)]), ref(31.0, 1.0, 1.0)) < 1e-13
+
+
+def _timed(ctx, f):
+    """The classes of the kernels that f launches."""
+    ctx.timing_report()
+    ctx.timing(True)
+    f()
+    ctx.timing(False)
+    return ctx.timing_report()
+
+
+def test_element_scatter_of_long_rows(gpu_ctx):
+    """A row whose 250 entries of 20 values are more than LDS takes: the elements are scattered colour by
+    colour, also in a call of 33 terms that adds to the first 32 (against the oracle as above)."""
+    C = core()
+    hm = fan(250)
+    fes = C.FESpace(C.Mesh(hm, gpu_ctx), [C.H1(3), C.H1(3)])
+    t = fem.Topology(hm)
+    cs = fem.Compound([fem.Space(t, 'H1', 3), fem.Space(t, 'H1', 3)])
+    for n in (1, 31):
+        a = C.BilinearForm(fes, [C.Vol('gradgrad', 0, 0, coef=2.0)] * n + [C.Vol('mass', 1, 1, coef=3.0),
+                                                                           C.Vol('mass', 1, 0, coef=0.5)])
+        assert 'assemble_h1_gather' not in _timed(gpu_ctx, a.Assemble)
+        A = fem.Assembler(cs)
+        fem.assemble_volume(A, [dict(kind='grad_grad', trial=0, test=0, coef=2.0 * n),
+                                dict(kind='mass', trial=1, test=1, coef=3.0),
+                                dict(kind='mass', trial=1, test=0, coef=0.5)])
+        assert rel(a.values(), A.matrix().data) < 1e-13
 
 
 def _field_case(C, ctx, gm, hm, t, order, seed, ncomp=1):
@@ -562,3 +590,94 @@ def test_kept_plans_follow_the_form(gpu_ctx):
     assert torch.equal(f.vec, b1)
     # twice the source is twice the vector, to the rounding of its sums
     assert float((f2.vec - 2 * b1).abs().max()) <= 1e-15 * float(b1.abs().max()) * 8
+
+
+def test_kept_plans_follow_what_changes(gpu_ctx):
+    """The same form assembled again after a coefficient, the contents of a per-element coefficient, the
+    values of a wind or a weight or the weighting field itself changed: bit for bit what a new form of the
+    same terms gives, and not what it gave before."""
+    import torch
+    C = core()
+    hm = unit_square(6)
+    gm = C.Mesh(hm, gpu_ctx)
+    fes = C.FESpace(gm, [C.H1(2)])
+    wind, w1, w2 = (C.GridFunction(C.FESpace(gm, [C.H1(p, ncomp=c)])) for p, c in ((2, 2), (1, 1), (2, 1)))
+    rng = np.random.default_rng(5)
+
+    def fill(v):
+        v.copy_(torch.from_numpy(rng.random(v.numel())).to(v.device))
+
+    kappa = torch.empty(hm.nel, dtype=torch.float64, device='cuda')
+    for v in (kappa, wind.vec, w1.vec, w2.vec):
+        fill(v)
+    terms = [C.Vol('gradgrad', 0, 0, elem_coef=kappa),
+             C.Vol('conv', 0, 0, wind_gf=(wind, wind.space.comp_blocks[0])),
+             C.Vol('mass', 0, 0, coef=2.0, weight_gf=(w1, 0, L.WEIGHT_FIELD)),
+             C.Vol('mass', 0, 0, coef=0.5, weight_gf=(w2, 0, L.WEIGHT_ONE_MINUS_FIELD))]
+    # alone, and as the last of 33 terms, which are added in a second launch
+    for terms in (terms, [C.Vol('gradgrad', 0, 0, elem_coef=kappa)] * 32 + terms[2:]):
+        a = C.BilinearForm(fes, terms)
+        a.Assemble()
+        last = a.values()
+
+        def again():
+            nonlocal last
+            a.Assemble()
+            fresh = C.BilinearForm(fes, list(terms))
+            fresh.Assemble()
+            assert np.array_equal(a.values(), fresh.values()) and not np.array_equal(a.values(), last)
+            last = a.values()
+
+        terms[-1].coef += 1.25
+        again()
+        for v in (kappa, w1.vec, w2.vec):
+            fill(v)
+            again()
+        if len(terms) == 4:
+            fill(wind.vec)
+            again()
+        terms[-1].weight_gf = (w1, 0, L.WEIGHT_ONE_MINUS_FIELD)
+        again()
+        terms[-1].weight_gf = (w2, 0, L.WEIGHT_FIELD)
+        again()
+
+
+def test_kept_load_plans_follow_what_changes(gpu_ctx):
+    """As above for load vectors, and with more of them in turn (12) than a space keeps plans (8)."""
+    import torch
+    C = core()
+    hm = unit_square(6)
+    gm = C.Mesh(hm, gpu_ctx)
+    fes = C.FESpace(gm, [C.H1(2)])
+    g, w = (C.GridFunction(C.FESpace(gm, [C.H1(p)])) for p in (2, 1))
+    rng = np.random.default_rng(6)
+
+    def fill(v):
+        v.copy_(torch.from_numpy(rng.random(v.numel())).to(v.device))
+
+    fill(g.vec)
+    fill(w.vec)
+    forms = [C.LinearForm(fes, [C.Source(0, field_gf=(g, 0), coef=1.0 + k, weight_gf=(w, 0, L.WEIGHT_FIELD)),
+                                C.Source(0, (L.FN_CONST, (0.1 * k,)))]) for k in range(12)]
+
+    def vectors(fs):
+        for f in fs:
+            f.Assemble()
+        return [f.vec.clone() for f in fs]
+
+    last = vectors(forms)
+    for change in ('field', 'weight', 'coefficient', 'source'):
+        if change == 'field':
+            fill(g.vec)
+        elif change == 'weight':
+            fill(w.vec)
+        for f in forms:
+            if change == 'coefficient':
+                f.terms[0].coef += 0.25
+            elif change == 'source':
+                f.terms[1].fn = (L.FN_CONST, (f.terms[1].fn[1][0] + 1.0,))
+        now = vectors(forms)
+        fresh = vectors([C.LinearForm(fes, list(f.terms)) for f in reversed(forms)])[::-1]
+        for a, b, c in zip(now, fresh, last):
+            assert torch.equal(a, b) and not torch.equal(a, c)
+        last = now

@@ -196,7 +196,9 @@ def test_learned_guess_saves_outer_iterations_with_schur_inner_solve(gpu_ctx):
     trained on them (base 1), then the same 4 steps from the same state with and without the learned
     guess. The guess wins the residual comparison on every step and the first Picard solve of each
     step needs fewer outer FGMRES iterations in total (the bench measures the same at n=228:
-    645 against 708 outer iterations over 5 steps)."""
+    645 against 708 outer iterations over 5 steps). The restarts make the count of one run depend on its
+    rounding (355 to 411 plain over six starts 1e-13 apart, 297 to 344 learned over five of them and six
+    trainings), so the totals of three starts are compared: 1,097 against 922."""
     from opencmp_amd.learned import GuessPolicy, MLPGuess
     from opencmp_amd.mesh import channel_with_holes
     from opencmp_amd.models import INS, const
@@ -229,12 +231,12 @@ def test_learned_guess_saves_outer_iterations_with_schur_inner_solve(gpu_ctx):
     wind = m0.W.vec.clone()
     del s0, m0, pol
 
-    def run(use_net):
+    def run(use_net, eps):
         m = model('mixed')
         p = GuessPolicy(gpu_ctx, n, net=net if use_net else None, n_learned=seg[-1])
         for h in reversed(ring[1:]):
             p.push(h)
-        s = ImplicitEulerSolver(m, dt=1e-3, gfu0=type(m.W)(m.fes, state.clone()), guess=p)
+        s = ImplicitEulerSolver(m, dt=1e-3, gfu0=type(m.W)(m.fes, state * (1.0 + eps)), guess=p)
         m.W.vec.copy_(wind)
         first, total = [], 0
         for _ in range(4):
@@ -244,12 +246,16 @@ def test_learned_guess_saves_outer_iterations_with_schur_inner_solve(gpu_ctx):
             total += m.linear_iterations
         return first, total, s.guess_log, s.gfu_prev.vec.clone()
 
-    fp, tp, _, up = run(False)
-    fl, tl, log, ul = run(True)
-    say(f'  first Picard solves: plain {fp} (total {tp}), learned {fl} (total {tl})')
-    say('  choices', [(c, f'{rp:.2e}', f'{rl:.2e}') for c, rp, rl in log])
-    assert all(c == 'learned' and rl < rp for c, rp, rl in log)
-    assert sum(fl) < sum(fp)
+    its = {False: 0, True: 0}
+    for eps in (2e-13, 1e-13, 0.0):
+        fp, tp, _, up = run(False, eps)
+        fl, tl, log, ul = run(True, eps)
+        say(f'  first Picard solves: plain {fp} (total {tp}), learned {fl} (total {tl})')
+        say('  choices', [(c, f'{rp:.2e}', f'{rl:.2e}') for c, rp, rl in log])
+        assert all(c == 'learned' and rl < rp for c, rp, rl in log)
+        its[False] += sum(fp)
+        its[True] += sum(fl)
+    assert its[True] < its[False]
     rel = float(torch.linalg.norm(ul - up) / torch.linalg.norm(up))
     say('  rel diff of the final states', rel)
     assert rel < 1e-2
