@@ -1358,10 +1358,11 @@ void build_h1_gather(Matrix *A) {
   int maxent = 0;
   for (int64_t r = 0; r < n; ++r) maxent = std::max(maxent, pptr[r + 1] - pptr[r]);
   // row blocks: staged values and their list (10 bytes each) of about 24 KB, greedily over
-  // consecutive rows (12, 16, 24 and 40 KB: 767, 626, 565 and 709 us on 62M 3D P3 nonzeros, 597, 605,
-  // 600 and 748 on 53M of the INS channel, 570, 414, 400 and 528 on 20M of 3D diffuse-interface
-  // Stokes); a row that alone exceeds that gets a block of its own and the buffers grow to it, up to
-  // 48 KB of LDS in all
+  // consecutive rows. An assembly with 12, 16, 20, 24, 32 and 40 KB: 62M nonzeros of 3D P3 763, 629, 541, 576, 693 and
+  // 715 us, 53M of the INS channel 810, 817, 754, 814, 960 and 947, 20M of 3D diffuse-interface Stokes 600,
+  // 450, 431, 442, 505 and 516, 6M of 2D P3 41, 37, 39, 45, 53 and 49, 1M of 3D P1 62, 62, 64, 71, 79 and 88: 24 KB was
+  // taken from the first three without 20, which is the better by 2 to 10 %. A row that alone exceeds it
+  // gets a block of its own and the buffers grow to it, up to 48 KB of LDS in all
   const int emax = std::max(std::max(1, 24576 / (nl * 10)), maxent);
   A->gemax = emax;
   A->npatch = np;
@@ -1454,8 +1455,10 @@ void build_h1_schedule(Matrix *A) {
   Space &s = *A->space;
   Mesh &m = *s.mesh;
   const int nl = s.nloc;
-  // element -> CSR slot map
-  std::vector<int32_t> slot((size_t)m.nel * nl * nl);
+  // element -> CSR slot map (first touched by the threads that fill it: 356 MB on the channel at n = 228, and
+  // cleared by one thread they were half of a form's first assembly: 115 ms, 60 now)
+  const size_t ns = (size_t)m.nel * nl * nl;
+  const std::unique_ptr<int32_t[]> slot(new int32_t[ns]);
 #pragma omp parallel for schedule(static)
   for (int64_t e = 0; e < m.nel; ++e) {
     const int32_t *ed = &s.edofs[e * nl];
@@ -1469,7 +1472,7 @@ void build_h1_schedule(Matrix *A) {
       }
     }
   }
-  A->d_slot.upload(slot, A->ctx->stream);
+  A->d_slot.upload(slot.get(), ns, A->ctx->stream);
   OCMP_HIP(hipStreamSynchronize(A->ctx->stream));
 }
 
