@@ -208,8 +208,8 @@ __global__ __launch_bounds__(NT) void k_conv3(Conv c) {
 // as the fourth such group, the bias), its wavefronts quarters of the chunk: each lane loads four
 // consecutive voxels of channel a = l % 16 once and the shifted voxels of channel b = l % 16 for
 // every tap, and v_mfma_f32_16x16x4 contracts voxel by voxel. Fixed partitions and order of sums.
-// 33^3 grid: 62 us (95 with a branch around each load) and 20 for the sums, against 426 us in 32 launches (one
-// per layer, operand and stage, on the vector units).
+// 33^3 grid: 64 us (95 with a branch around each load) and 8 for the sums over the chunks (20 with one load in
+// flight), against 426 us in 32 launches (one per layer, operand and stage, on the vector units).
 struct WGrad {
   const void *P, *Q, *G;
   int p_bf16, na, np, q_bf16, nb, nq, stride;
@@ -222,9 +222,10 @@ struct WGrads {
   WGrad l[NL];
 };
 
-// A chunk grows with the grid beyond 256 of them (from 53^3 voxels on): a wavefront's FP32 sums run over at most WG_RUN
-// tiles of 16 voxels and are then added up, so that a sum of 129^3 products is 128 + 17 additions long and
-// not 2,096; the partial sums of the chunks and the biases are summed in FP64.
+// A chunk grows with the grid beyond 256 of them (from 53^3 voxels on): a wavefront's FP32 sums run over at
+// most WG_RUN tiles of 16 voxels and are then added up in LDS, so that a sum of 129^3 products is 128 + 17
+// additions long and not 2,096; the partial sums of the chunks and the biases are summed in FP64. (Added up in
+// registers: two waves a SIMD instead of three, 33^3 203 -> 213 us a gradient; in LDS 192.)
 constexpr int WG_RUN = 8;
 
 __device__ __forceinline__ int64_t chunk_len(int64_t n, int nch) { return ((n + nch - 1) / nch + 15) / 16 * 16; }
